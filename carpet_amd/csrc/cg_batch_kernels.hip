@@ -40,7 +40,7 @@ namespace cg {
 #ifndef CG_POINT_NT
 #define CG_POINT_NT 1
 #endif
-__device__ __forceinline__ void point_store(double v, double *p) {
+__device__ __forceinline__ void point_store(double v, gdst_t p) {
   if constexpr (CG_POINT_NT)
     __builtin_nontemporal_store(v, p);
   else
@@ -150,7 +150,7 @@ __device__ __forceinline__ void point_item(const PointArgs &a, unsigned tile, in
 #pragma unroll
       for (int u = 0; u < PU; ++u)
         if (o[u] >= 0)
-          point_store(v[u], a.dst + o[u]);
+          point_store(v[u], (gdst_t)a.dst + o[u]);
     }
   }
 }
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(256) void k_grid_point_n(const PointArgs *__restric
   const int x = blockIdx.x & 7;
   const int i0 = seg[x] + (int)(blockIdx.x >> 3) * NI, i1 = seg[x + 1];
   double v[NI];
-  double *q[NI]; // destination of each value, null outside the item
+  gdst_t q[NI]; // destination of each value, null outside the item
 #pragma unroll
   for (int u = 0; u < NI; ++u) {
     q[u] = nullptr;
@@ -212,7 +212,7 @@ __global__ __launch_bounds__(256) void k_grid_point_n(const PointArgs *__restric
         const unsigned j = fastdiv(r, a.fx);
         const unsigned i = r - j * nx;
         v[u] = point_value<OP>(a, (int)i, (int)j, (int)k);
-        q[u] = a.dst + ((long long)i + a.dj * j + a.dk * k);
+        q[u] = (gdst_t)a.dst + ((long long)i + a.dj * j + a.dk * k);
       }
     }
   }
@@ -583,14 +583,16 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     // per step against 19.43 ms with 4096)
     else if (g.op == PO_COPY)
       l.pt = 2048;
-    // tensor tiles of large regions (median 2^20 points and up): persistent
-    // grid (its workgroups take the tiles in order, so neighbouring tiles
-    // march through z together and share halo rows in L2); other tensor
-    // classes and pointwise runs: one workgroup per item.  (Measured: on
-    // 2000 regions of 8-96 points per axis both modes are within 0.2%; on a
-    // hierarchy's shells one workgroup per item takes 0.45 ms less per
-    // step for the small tiles and 0.09 ms less for the large ones.)
-    l.wpc = g.is_tensor && !g.small && median_pts >= (1LL << 20) ? 0 : -1;
+    // tensor tiles of very large regions (median 2^25 points and up):
+    // persistent grid (its workgroups take the tiles in order, so
+    // neighbouring tiles march through z together and share halo rows in
+    // L2); other tensor classes and pointwise runs: one workgroup per item.
+    // (Measured, persistent against one per item: 4 x 512^3 order 5, 3
+    // levels 1.35 against 1.38 ms; 8 x 384^3 with FP32 storage 633 against
+    // 642 us; 8 x 320^3 cell ENO<3> equal; 5 x 256^3 vertex ENO, 3 levels,
+    // 378 against 323 us; 8 x 231x165x297 order 3, 2 levels, 240 against
+    // 216 us.)
+    l.wpc = g.is_tensor && !g.small && median_pts >= (1LL << 25) ? 0 : -1;
     // tile shape: the class's (its regions were routed by shape)
     l.shape = !g.is_tensor ? 0 : g.small ? g.small : g.bigsh;
     if (tuned) {

@@ -46,7 +46,8 @@ __attribute__((amdgpu_waves_per_eu(persist_waves<L, NTL, CX, CY, IPT>()))) void 
 }
 
 template <class L, int NTL, int CX, int CY, int IPT, int XQ, int PR, int NSRC>
-__global__ __launch_bounds__(2 * CX * CY / IPT) void k_grid_tensor(
+__global__ __launch_bounds__(2 * CX * CY / IPT)
+__attribute__((amdgpu_waves_per_eu(persist_waves<L, NTL, CX, CY, IPT>()))) void k_grid_tensor(
     const TensorArgs *__restrict__ descs, const Item *__restrict__ items,
     const int *__restrict__ seg) {
   __shared__ __align__(16) double smem[tile_lds<L, NTL, CX, CY, XQ>()];
@@ -54,8 +55,8 @@ __global__ __launch_bounds__(2 * CX * CY / IPT) void k_grid_tensor(
   if (it < 0)
     return;
   const Item w = items[it];
-  tensor_tile<L, NTL, CX, CY, IPT, PR, BATCH_PF, XQ, pipe_fits<L, NTL, CX, CY, XQ>(), NSRC>(descs[w.desc],
-                                                                                            (int)w.tile, smem);
+  const TensorArgs a = descs[w.desc];
+  tensor_tile<L, NTL, CX, CY, IPT, PR, BATCH_PF, XQ, pipe_fits<L, NTL, CX, CY, XQ>(), NSRC>(a, (int)w.tile, smem);
 }
 
 template <class L, int NSRC, int PR, int SH>

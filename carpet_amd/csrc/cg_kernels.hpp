@@ -7,6 +7,22 @@
 
 namespace cg {
 
+// Array pointers reach the batch kernels through descriptors in memory, and
+// the compiler cannot tell that such a pointer is to global memory: its
+// accesses become flat ones, which also count as LDS operations, so every
+// wait for an LDS read waits for the global loads and stores in flight too.
+// Kernels therefore cast them: CG_GLOBAL T * is a pointer to global memory.
+// Batched, flat against global: 8 x 384^3 FP32-storage order-5 prolongations
+// 715 against 632 us, 8 x 320^3 cell ENO<3> 914 against 784 us, the level
+// step of 3 levels of 8 components 1.02 against 0.96 ms.
+#ifdef __HIP_DEVICE_COMPILE__
+#define CG_GLOBAL __attribute__((address_space(1)))
+#else
+#define CG_GLOBAL
+#endif
+using gsrc_t = CG_GLOBAL const double *;
+using gdst_t = CG_GLOBAL double *;
+
 // Tensor-product prolongation (Lagrange vertex/cell, ENO cell) fused with
 // time interpolation over up to 3 source time levels.
 struct TensorArgs {

@@ -52,10 +52,6 @@ __device__ __forceinline__ int xcd_remap(int b, int n) {
   return xcd * per + min(xcd, rem) + slot;
 }
 
-template <typename TS> __device__ __forceinline__ double ld(const void *p, long long o) {
-  return (double)(static_cast<const TS *>(p)[o]);
-}
-
 // LDS footprint (doubles) of one tensor tile; XQ = bases per thread in the
 // x-pass (2: rows padded to an even stride for 16-byte LDS accesses); NB =
 // buffers of the window and of the x-pass results (2 for the pipelined
@@ -222,7 +218,7 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
       if (woff[k] >= 0)
 #pragma unroll
         for (int tl = 0; tl < NSRC; ++tl)
-          pre[SL][tl][k] = static_cast<const TS *>(a.src[tl])[woff[k] + a.sk * c];
+          pre[SL][tl][k] = ((CG_GLOBAL const TS *)a.src[tl])[woff[k] + a.sk * c];
   };
 
   // ring of y-pass results: slot j holds the planes c with (c - c0) % R == j
@@ -347,7 +343,7 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
           // time interpolation in FP64 in every precision mode
           const double out = time_combine<NTL>(v, a.s, a.s2, a.l0, a.teno, a.nlev);
           if (xin && fy >= 0 && fy < a.n[1])
-            __builtin_nontemporal_store((TS)out, &static_cast<TS *>(a.dst)[gfx + a.dj * fy + a.dk * fz]);
+            __builtin_nontemporal_store((TS)out, &((CG_GLOBAL TS *)a.dst)[gfx + a.dj * fy + a.dk * fz]);
         }
       }
     };
@@ -423,10 +419,10 @@ __device__ __forceinline__ double minmod(double a, double b) {
 // product and sum rounded on its own; where the value leaves the range of
 // the 2, 4 or 8 nearest coarse values, their average (weights 1/2 per axis,
 // the same corner order) replaces it
-__device__ __forceinline__ double mono5_value(const double *src, long long J, long long K, int gi, int gj,
+__device__ __forceinline__ double mono5_value(gsrc_t src, long long J, long long K, int gi, int gj,
                                               int gk) {
   constexpr double f[6] = {3 / 256.0, -25 / 256.0, 150 / 256.0, 150 / 256.0, -25 / 256.0, 3 / 256.0};
-  const double *p = src + (gi >> 1) + J * (gj >> 1) + K * (gk >> 1);
+  const gsrc_t p = src + (gi >> 1) + J * (gj >> 1) + K * (gk >> 1);
   const int pi = gi & 1, pj = gj & 1, pk = gk & 1;
   const int nodd = pi + pj + pk;
   if (nodd == 0)
@@ -536,11 +532,11 @@ __device__ __forceinline__ double stag_coef(int order, int kind, int t) {
 // source array: sum from 0 of coeff_x * coeff_y * coeff_z * src, x taps
 // outermost and z innermost, each operation rounded as written (the
 // coefficient products are exact: dyadic numerators below 2^21)
-__device__ __forceinline__ double stagger_value(const double *src, long long J, long long K, int gi, int gj,
+__device__ __forceinline__ double stagger_value(gsrc_t src, long long J, long long K, int gi, int gj,
                                                 int gk, int stag, int order) {
   const int kx = stag_kind(stag, 0, gi & 1), ky = stag_kind(stag, 1, gj & 1), kz = stag_kind(stag, 2, gk & 1);
   const int nx = stag_n(order, kx), ny = stag_n(order, ky), nz = stag_n(order, kz);
-  const double *p = src + ((gi >> 1) + stag_lo(order, kx)) + J * ((gj >> 1) + stag_lo(order, ky)) +
+  const gsrc_t p = src + ((gi >> 1) + stag_lo(order, kx)) + J * ((gj >> 1) + stag_lo(order, ky)) +
                     K * ((gk >> 1) + stag_lo(order, kz));
   double r = 0.0;
 #pragma unroll
@@ -569,14 +565,14 @@ __device__ __forceinline__ double stagger_value(const double *src, long long J, 
 // coarse point's coincident child): staggered directions take fine points
 // 2i-1..2i+2 with {-1, 9, 9, -1}/16, unstaggered ones 2i-1..2i+1 with
 // {1, 6, 1}/8 (coeffs_restrict_3d_stagger.hh, ORDER_STAG 3)
-__device__ __forceinline__ double stagger_restrict_value(const double *p, long long J, long long K, int stag) {
+__device__ __forceinline__ double stagger_restrict_value(gsrc_t p, long long J, long long K, int stag) {
   auto coef = [](int s, int t) -> double {
     if (s)
       return t == 0 || t == 3 ? -1.0 / 16.0 : 9.0 / 16.0;
     return t == 1 ? 6.0 / 8.0 : 1.0 / 8.0;
   };
   const int sx = stag & 1, sy = (stag >> 1) & 1, sz = (stag >> 2) & 1;
-  const double *q = p - 1 - J - K;
+  const gsrc_t q = p - 1 - J - K;
   double r = 0.0;
 #pragma unroll
   for (int a = 0; a < 4; ++a) {
@@ -606,13 +602,14 @@ template <int OP>
 __device__ __forceinline__ double point_value(const PointArgs &a, int i, int j, int k) {
   static_assert(OP != PO_TVD, "TVD runs per coarse cell (tvd_cell)");
   double out;
+  const auto src = [&](int l) { return (gsrc_t)a.src[l]; };
   if constexpr (OP == PO_COPY) {
-    out = a.src[0][i + a.sj * j + a.sk * k];
+    out = src(0)[i + a.sj * j + a.sk * k];
   } else if constexpr (OP == PO_RESTRICT_VC) {
-    out = a.src[0][2 * i + a.sj * (2 * j) + a.sk * (2 * k)];
+    out = src(0)[2 * i + a.sj * (2 * j) + a.sk * (2 * k)];
   } else if constexpr (OP == PO_RESTRICT_CC) {
     // restrict_3d_cc_rf2.cc:118-126: eight children, fixed order, weight 1/8
-    const double *p = a.src[0] + 2 * i + a.sj * (2 * j) + a.sk * (2 * k);
+    const gsrc_t p = src(0) + 2 * i + a.sj * (2 * j) + a.sk * (2 * k);
     const long long J = a.sj, K = a.sk;
     const double w = (1.0 / 2) * (1.0 / 2) * (1.0 / 2);
     double r = w * p[0];
@@ -628,15 +625,15 @@ __device__ __forceinline__ double point_value(const PointArgs &a, int i, int j, 
     // each time level prolongated, then combined in time (data.cc:497-521)
     const int gi = a.off[0] + i, gj = a.off[1] + j, gk = a.off[2] + k;
     double v[3];
-    v[0] = mono5_value(a.src[0], a.sj, a.sk, gi, gj, gk);
+    v[0] = mono5_value(src(0), a.sj, a.sk, gi, gj, gk);
     if (a.ntl == 1) {
       out = v[0];
     } else {
-      v[1] = mono5_value(a.src[1], a.sj, a.sk, gi, gj, gk);
+      v[1] = mono5_value(src(1), a.sj, a.sk, gi, gj, gk);
       if (a.ntl == 2) {
         out = time_combine<2>(v, a.s, a.s2, a.l0, 0);
       } else {
-        v[2] = mono5_value(a.src[2], a.sj, a.sk, gi, gj, gk);
+        v[2] = mono5_value(src(2), a.sj, a.sk, gi, gj, gk);
         out = time_combine<3>(v, a.s, a.s2, a.l0, a.teno);
       }
     }
@@ -644,15 +641,15 @@ __device__ __forceinline__ double point_value(const PointArgs &a, int i, int j, 
     // each time level prolongated, then combined in time (data.cc:497-521)
     const int gi = a.off[0] + i, gj = a.off[1] + j, gk = a.off[2] + k;
     double v[3];
-    v[0] = stagger_value(a.src[0], a.sj, a.sk, gi, gj, gk, a.stag, a.sorder);
+    v[0] = stagger_value(src(0), a.sj, a.sk, gi, gj, gk, a.stag, a.sorder);
     if (a.ntl == 1) {
       out = v[0];
     } else {
-      v[1] = stagger_value(a.src[1], a.sj, a.sk, gi, gj, gk, a.stag, a.sorder);
+      v[1] = stagger_value(src(1), a.sj, a.sk, gi, gj, gk, a.stag, a.sorder);
       if (a.ntl == 2) {
         out = time_combine<2>(v, a.s, a.s2, a.l0, 0);
       } else {
-        v[2] = stagger_value(a.src[2], a.sj, a.sk, gi, gj, gk, a.stag, a.sorder);
+        v[2] = stagger_value(src(2), a.sj, a.sk, gi, gj, gk, a.stag, a.sorder);
         out = time_combine<3>(v, a.s, a.s2, a.l0, 0);
       }
     }
@@ -661,17 +658,17 @@ __device__ __forceinline__ double point_value(const PointArgs &a, int i, int j, 
     // cell-centred direction (bit of a.stag) averages its two children, a
     // vertex-centred one takes the first; the halves are exact, so each
     // half*a + half*b is one rounding however it is contracted
-    const double *p = a.src[0] + 2 * i + a.sj * (2 * j) + a.sk * (2 * k);
+    const gsrc_t p = src(0) + 2 * i + a.sj * (2 * j) + a.sk * (2 * k);
     const int cm = a.stag;
-    auto r1 = [&](const double *q) { return (cm & 1) ? 0.5 * q[0] + 0.5 * q[1] : q[0]; };
-    auto r2 = [&](const double *q) { return (cm & 2) ? 0.5 * r1(q) + 0.5 * r1(q + a.sj) : r1(q); };
+    auto r1 = [&](gsrc_t q) { return (cm & 1) ? 0.5 * q[0] + 0.5 * q[1] : q[0]; };
+    auto r2 = [&](gsrc_t q) { return (cm & 2) ? 0.5 * r1(q) + 0.5 * r1(q + a.sj) : r1(q); };
     out = (cm & 4) ? 0.5 * r2(p) + 0.5 * r2(p + a.sk) : r2(p);
   } else if constexpr (OP == PO_RESTRICT_STAGGER) {
-    out = stagger_restrict_value(a.src[0] + 2 * i + a.sj * (2 * j) + a.sk * (2 * k), a.sj, a.sk, a.stag);
+    out = stagger_restrict_value(src(0) + 2 * i + a.sj * (2 * j) + a.sk * (2 * k), a.sj, a.sk, a.stag);
   } else if constexpr (OP == PO_RESTRICT_CC_O3) {
     // restrict_3d_cc_o3_rf2.cc:146-211: 64 terms, (w_a w_b w_c)/4096 with
     // w = {-1, 9, 9, -1}, a fastest, then b, then c; fine cells 2i-1..2i+2
-    const double *p = a.src[0] + 2 * i + a.sj * (2 * j) + a.sk * (2 * k);
+    const gsrc_t p = src(0) + 2 * i + a.sj * (2 * j) + a.sk * (2 * k);
     constexpr double w[4] = {-1, 9, 9, -1};
     double r = 0.0;
 #pragma unroll
@@ -688,7 +685,7 @@ __device__ __forceinline__ double point_value(const PointArgs &a, int i, int j, 
   } else if constexpr (OP == PO_RESTRICT_CC_O5) {
     // restrict_3d_cc_o5_rf2.cc:36-74: 6-point sums, x inside y inside z,
     // weights {3, -25, 150, 150, -25, 3}/256; fine cells 2i-2..2i+3
-    const double *p = a.src[0] + 2 * i + a.sj * (2 * j) + a.sk * (2 * k);
+    const gsrc_t p = src(0) + 2 * i + a.sj * (2 * j) + a.sk * (2 * k);
     constexpr double w[6] = {3.0 / 256, -25.0 / 256, 150.0 / 256, 150.0 / 256, -25.0 / 256, 3.0 / 256};
     double r2 = 0.0;
 #pragma unroll
@@ -696,7 +693,7 @@ __device__ __forceinline__ double point_value(const PointArgs &a, int i, int j, 
       double r1 = 0.0;
 #pragma unroll
       for (int b = 0; b < 6; ++b) {
-        const double *q = p + a.sj * (b - 2) + a.sk * (c - 2);
+        const gsrc_t q = p + a.sj * (b - 2) + a.sk * (c - 2);
         double x = w[0] * q[-2];
 #pragma unroll
         for (int aa = 1; aa < 6; ++aa)
@@ -710,22 +707,22 @@ __device__ __forceinline__ double point_value(const PointArgs &a, int i, int j, 
     const long long o = i + a.sj * j + a.sk * k;
     if (a.ntl > 3) {
       // interpolate_3d_4tl / _5tl: s1*a, then fma(s_l, level l, .)
-      double r = a.s[0] * a.src[0][o];
-      r = fmad(a.s[1], a.src[1][o], r);
-      r = fmad(a.s[2], a.src[2][o], r);
-      r = fmad(a.s[3], a.src[3][o], r);
+      double r = a.s[0] * src(0)[o];
+      r = fmad(a.s[1], src(1)[o], r);
+      r = fmad(a.s[2], src(2)[o], r);
+      r = fmad(a.s[3], src(3)[o], r);
       if (a.ntl == 5)
-        r = fmad(a.s[4], a.src[4][o], r);
+        r = fmad(a.s[4], src(4)[o], r);
       out = r;
     } else if (a.ntl == 3) {
-      const double v[3] = {a.src[0][o], a.src[1][o], a.src[2][o]};
+      const double v[3] = {src(0)[o], src(1)[o], src(2)[o]};
       out = time_combine<3>(v, a.s, a.s2, a.l0, a.teno);
     } else if (a.ntl == 1) {
       // a batched same-level interpolation whose target time has become an
       // exact match: the copy of that level
-      out = a.src[0][o];
+      out = src(0)[o];
     } else {
-      const double v[2] = {a.src[0][o], a.src[1][o]};
+      const double v[2] = {src(0)[o], src(1)[o]};
       out = time_combine<2>(v, a.s, a.s2, a.l0, a.teno);
     }
   }
@@ -734,7 +731,7 @@ __device__ __forceinline__ double point_value(const PointArgs &a, int i, int j, 
 
 template <int OP>
 __device__ __forceinline__ void point_elem(const PointArgs &a, int i, int j, int k) {
-  a.dst[i + a.dj * j + a.dk * k] = point_value<OP>(a, i, j, k);
+  ((gdst_t)a.dst)[i + a.dj * j + a.dk * k] = point_value<OP>(a, i, j, k);
 }
 
 // Cell-centred TVD prolongation (prolongate_3d_cc_real8_tvd.F90:183-225)
@@ -758,7 +755,7 @@ struct TvdCell {
 };
 __device__ __forceinline__ TvdCell tvd_load(const PointArgs &a, int tl, int qx, int qy, int qz) {
   const long long J = a.sj, K = a.sk;
-  const double *p = a.src[tl] + qx + J * qy + K * qz;
+  const gsrc_t p = (gsrc_t)a.src[tl] + qx + J * qy + K * qz;
   const double c = p[0];
   return TvdCell{c, minmod(c - p[-1], p[1] - c), minmod(c - p[-J], p[J] - c),
                  minmod(c - p[-K], p[K] - c)};
@@ -793,13 +790,13 @@ __device__ __forceinline__ void tvd_store(const PointArgs &a, int qx, int qy, in
         }
         out[x] = time_combine<NTL>(w, a.s, a.s2, a.l0, a.teno);
       }
-      double *p = &a.dst[fx0 + a.dj * fy + a.dk * fz];
+      const gdst_t p = (gdst_t)a.dst + (fx0 + a.dj * fy + a.dk * fz);
       const bool in0 = fx0 >= 0 && fx0 < a.n[0], in1 = fx0 + 1 >= 0 && fx0 + 1 < a.n[0];
       // both x children in one 16-byte store where the pair is aligned, so a
       // wavefront writes whole contiguous lines (two 8-byte stores per lane
       // at a 16-byte stride leave every line half written per instruction)
-      if (in0 && in1 && ((reinterpret_cast<uintptr_t>(p) & 15) == 0)) {
-        __builtin_nontemporal_store(dbl2{out[0], out[1]}, reinterpret_cast<dbl2 *>(p));
+      if (in0 && in1 && (((uintptr_t)p & 15) == 0)) {
+        __builtin_nontemporal_store(dbl2{out[0], out[1]}, (CG_GLOBAL dbl2 *)p);
       } else {
         if (in0)
           __builtin_nontemporal_store(out[0], p);

@@ -257,7 +257,7 @@ struct Group {
 double tile_busy(const TensorArgs &a, int ntl, int prec, int span, int sh) {
   int cx, cy, th;
   tile_shape(ntl, prec, &cx, &cy, &th, sh);
-  return (double)((a.nq[0] + cx - 1) / cx) * ((a.nq[1] + cy - 1) / cy) * (a.nq[2] + span) * cx *
+  return (double)tiles_x(a, cx, tile_shift(a, cx, prec ? 4 : 8)) * ((a.nq[1] + cy - 1) / cy) * (a.nq[2] + span) * cx *
          (cy + span);
 }
 
@@ -299,14 +299,16 @@ int small_tiles(const ProlongPlan &p, int ntl, int prec) {
 // more levels keeps nlev = 1 and reads level 0 for every level slot; a
 // same-level interpolation resolved to a copy stays an interpolation of one
 // level
-TensorArgs tensor_desc(const BatchLaunch &l, const Transfer &t) {
+TensorArgs tensor_desc(const BatchLaunch &l, const Transfer &t, int sx = -1) {
   TensorArgs a = t.pr.t;
   for (int k = a.nlev; k < l.ntl; ++k)
     a.src[k] = a.src[0];
+  a.sx = sx;
   TileCfg cfg;
   int th = 0;
   tile_shape(l.ntl, l.prec, &cfg.cx, &cfg.cy, &th, l.shape);
   cfg.zchunk = l.zchunk;
+  cfg.es = l.prec ? 4 : 8;
   (void)tensor_tiles(a, cfg);
   return a;
 }
@@ -452,7 +454,7 @@ void batch_launch_descs(const BatchLaunch &l, const std::vector<Transfer> &tr, c
   for (size_t i = 0; i < l.members.size(); ++i) {
     const Transfer &t = tr[l.members[i]];
     if (l.is_tensor) {
-      const TensorArgs a = tensor_desc(l, t);
+      const TensorArgs a = tensor_desc(l, t, l.sx[i]);
       std::memcpy(out + i * sizeof(TensorArgs), &a, sizeof a);
     } else {
       const PointArgs a = point_desc(l, t);
@@ -651,7 +653,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
           for (int m : members) {
             const TensorArgs &a = tr[m].pr.t;
             const long long nxy =
-                (long long)((a.nq[0] + cfg.cx - 1) / cfg.cx) * ((a.nq[1] + cfg.cy - 1) / cfg.cy);
+                (long long)tiles_x(a, cfg.cx, tile_shift(a, cfg.cx, g.prec ? 4 : 8)) * ((a.nq[1] + cfg.cy - 1) / cfg.cy);
             for (int z0 = 0; z0 < a.nq[2]; z0 += zc)
               for (long long t = 0; t < nxy; ++t) {
                 const double at = q.top();
@@ -682,6 +684,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
         const long long nt = (long long)a.ntiles[0] * a.ntiles[1] * a.ntiles[2];
         const unsigned d = (unsigned)descs.size();
         descs.push_back(a);
+        l.sx.push_back(a.sx);
         first.push_back((int)items.size());
         for (long long t = 0; t < nt; ++t) {
           items.push_back(Item{d, (unsigned)t});

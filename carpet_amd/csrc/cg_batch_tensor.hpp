@@ -26,12 +26,12 @@ constexpr int BATCH_PF = 1;
 
 // NTL: levels of the passes; NSRC: source levels (NSRC > NTL: combined at
 // the window store)
-template <class L, int NTL, int CX, int CY, int IPT, int XQ, int PR, int NSRC>
+template <class L, int NTL, int CX, int CY, int IPT, int PR, int NSRC>
 __global__ __launch_bounds__(2 * CX * CY / IPT)
 __attribute__((amdgpu_waves_per_eu(persist_waves<L, NTL, CX, CY, IPT>()))) void k_persist_tensor(
     const TensorArgs *__restrict__ descs, const Item *__restrict__ items,
     const int *__restrict__ seg, int *counter, int stat) {
-  __shared__ __align__(16) double smem[tile_lds<L, NTL, CX, CY, XQ>()];
+  __shared__ __align__(16) double smem[tile_lds<L, NTL, CX, CY>()];
   __shared__ int s_item;
   for (int k = 0;; ++k) {
     // stat: fixed rounds over the XCD's segment, else the work counters
@@ -40,23 +40,23 @@ __attribute__((amdgpu_waves_per_eu(persist_waves<L, NTL, CX, CY, IPT>()))) void 
       return;
     const Item w = items[it];
     const TensorArgs a = descs[w.desc];
-    tensor_tile<L, NTL, CX, CY, IPT, PR, BATCH_PF, XQ, pipe_fits<L, NTL, CX, CY, XQ>(), NSRC>(a, (int)w.tile,
+    tensor_tile<L, NTL, CX, CY, IPT, PR, BATCH_PF, pipe_fits<L, NTL, CX, CY>(), NSRC>(a, (int)w.tile,
                                                                                           smem);
   }
 }
 
-template <class L, int NTL, int CX, int CY, int IPT, int XQ, int PR, int NSRC>
+template <class L, int NTL, int CX, int CY, int IPT, int PR, int NSRC>
 __global__ __launch_bounds__(2 * CX * CY / IPT)
 __attribute__((amdgpu_waves_per_eu(persist_waves<L, NTL, CX, CY, IPT>()))) void k_grid_tensor(
     const TensorArgs *__restrict__ descs, const Item *__restrict__ items,
     const int *__restrict__ seg) {
-  __shared__ __align__(16) double smem[tile_lds<L, NTL, CX, CY, XQ>()];
+  __shared__ __align__(16) double smem[tile_lds<L, NTL, CX, CY>()];
   const int it = grid_item(seg);
   if (it < 0)
     return;
   const Item w = items[it];
   const TensorArgs a = descs[w.desc];
-  tensor_tile<L, NTL, CX, CY, IPT, PR, BATCH_PF, XQ, pipe_fits<L, NTL, CX, CY, XQ>(), NSRC>(a, (int)w.tile, smem);
+  tensor_tile<L, NTL, CX, CY, IPT, PR, BATCH_PF, pipe_fits<L, NTL, CX, CY>(), NSRC>(a, (int)w.tile, smem);
 }
 
 template <class L, int NSRC, int PR, int SH>
@@ -66,10 +66,10 @@ int batch_tensor_go(const BatchLaunch &l, const TensorArgs *td, const Item *item
   using T = TileShape<NTL, SH, PR>;
   const dim3 block(tile_threads<NTL, SH, PR>());
   if (l.wpc == -1)
-    hipLaunchKernelGGL((k_grid_tensor<L, NTL, T::CX, T::CY, T::IPT, T::XQ, PR, NSRC>), dim3(l.grid), block,
+    hipLaunchKernelGGL((k_grid_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC>), dim3(l.grid), block,
                        0, st, td, items, seg);
   else
-    hipLaunchKernelGGL((k_persist_tensor<L, NTL, T::CX, T::CY, T::IPT, T::XQ, PR, NSRC>), dim3(l.grid),
+    hipLaunchKernelGGL((k_persist_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC>), dim3(l.grid),
                        block, 0, st, td, items, seg, ctr, l.wpc == -2 ? 1 : 0);
   return 0;
 }
@@ -111,7 +111,7 @@ template <int KIND, int SH> const void *batch_tensor_fn_kind(const BatchLaunch &
       constexpr int NTL = pass_levels(NSRC, PR);
       using T = TileShape<NTL, SH, PR>;
       *threads = tile_threads<NTL, SH, PR>();
-      fn = reinterpret_cast<const void *>(&k_persist_tensor<L, NTL, T::CX, T::CY, T::IPT, T::XQ, PR, NSRC>);
+      fn = reinterpret_cast<const void *>(&k_persist_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC>);
     };
     auto by_prec = [&](auto ntlc) {
       if (l.prec == 0)

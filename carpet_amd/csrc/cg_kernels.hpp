@@ -38,6 +38,8 @@ struct TensorArgs {
   int qlo[3];         // first coarse base (off>>1)
   int nq[3];          // number of coarse bases per axis
   int ntiles[3];      // tile counts: x, y (in CX/CY bases), z (chunks)
+  int sx;             // the tile grid starts sx fine columns before the region
+                      // (tensor_tiles; < 0: not chosen yet)
   int zchunk;         // coarse bases per z chunk
   double s[3];        // time weights
   double s2[2];       // ENO time rule: weights of the fallback pair
@@ -97,6 +99,7 @@ struct PointArgs {
 struct TileCfg {
   int cx, cy; // coarse bases per tile in x and y (fine tile 2cx x 2cy)
   int zchunk; // coarse bases per z chunk
+  int es;     // bytes per element of the arrays
 };
 
 // ---- launchers (defined in cg_kernels.hip) --------------------------------
@@ -109,7 +112,12 @@ int launch_tensor_kind(int order, int ntl, int prec, const TensorArgs &a, const 
                        hipStream_t s);
 int launch_tensor(int kind, int order, int ntl, int prec, const TensorArgs &a,
                   const TileCfg &cfg, hipStream_t s);
-// computes ntiles/zchunk of a for a tile configuration; returns block count
+// columns by which the tile grid of width 2 * cx starts before region r of a,
+// and the tiles along x that follow from it
+int tile_shift(const TensorArgs &a, int cx, int es);
+inline int tiles_x(const TensorArgs &a, int cx, int sx) { return (a.n[0] + sx + 2 * cx - 1) / (2 * cx); }
+// computes ntiles/zchunk (and sx, unless it is set) of a for a tile
+// configuration; returns block count
 long long tensor_tiles(TensorArgs &a, const TileCfg &cfg);
 int launch_point(int op, const PointArgs &a, hipStream_t s);
 int launch_fill(double *dst, double v, size_t n, hipStream_t s);

@@ -355,6 +355,7 @@ int plan_prolong(int kind, int order, const Arr &src, const void *const *srcs,
   for (int l = 0; l < 3; ++l)
     t.s[l] = l < ntl ? s[l] : 0.0;
   t.nlev = ntl;
+  t.sx = -1;
   if (eno && ntl == 3) {
     t.teno = 1;
     t.l0 = eno->l0;
@@ -376,14 +377,14 @@ int launch_prolong(const ProlongPlan &pl, int prec, hipStream_t st) {
   } else if (pl.kind == PK_STAGGER) {
     r = launch_point(PO_STAGGER, pl.p, st);
   } else {
-    TileCfg cfg{0, 0, 0};
+    TileCfg cfg{0, 0, 0, pl.es};
     // z chunks: at most 128 planes (tiles that march much further apart in
     // z stop sharing their halo rows through L2), at least 2^18 threads (a
     // full round of resident workgroups), at least 16 planes per chunk
     TensorArgs a = pl.t;
     int threads = 0;
     tile_shape(pl.ntl, prec, &cfg.cx, &cfg.cy, &threads);
-    const long long cols = (long long)((a.nq[0] + cfg.cx - 1) / cfg.cx) *
+    const long long cols = (long long)tiles_x(a, cfg.cx, tile_shift(a, cfg.cx, cfg.es)) *
                            ((a.nq[1] + cfg.cy - 1) / cfg.cy);
     int zc = std::min(a.nq[2], 128);
     while (zc > 16 && cols * ((a.nq[2] + zc - 1) / zc) * threads < (1LL << 18))

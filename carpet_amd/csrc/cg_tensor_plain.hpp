@@ -13,11 +13,11 @@ namespace cg {
 // the window store)
 // 512-thread workgroups of orders up to 5 held to 128 VGPRs, two per CU
 // (the O=5, 3-level tile otherwise takes 130 and runs one per CU)
-template <class L, int NTL, int CX, int CY, int IPT, int XQ, int PR, int NSRC>
+template <class L, int NTL, int CX, int CY, int IPT, int PR, int NSRC>
 __global__ __launch_bounds__(2 * CX * CY / IPT) __attribute__((amdgpu_waves_per_eu(
     (2 * CX * CY / IPT >= 512 && L::R <= 6) ? 4 : 1))) void k_tensor(TensorArgs a) {
-  __shared__ __align__(16) double smem[tile_lds<L, NTL, CX, CY, XQ>()];
-  tensor_tile<L, NTL, CX, CY, IPT, PR, 1, XQ, pipe_fits<L, NTL, CX, CY, XQ>(), NSRC>(
+  __shared__ __align__(16) double smem[tile_lds<L, NTL, CX, CY>()];
+  tensor_tile<L, NTL, CX, CY, IPT, PR, 1, pipe_fits<L, NTL, CX, CY>(), NSRC>(
       a, xcd_remap(blockIdx.x, gridDim.x), smem);
 }
 
@@ -32,7 +32,7 @@ int launch_tensor_t(const TensorArgs &a0, const TileCfg &cfg0, hipStream_t s) {
   const long long nblk = tensor_tiles(a, cfg);
   if (nblk <= 0 || nblk > 0x7fffffffLL)
     return -1;
-  hipLaunchKernelGGL((k_tensor<L, NTL, T::CX, T::CY, T::IPT, T::XQ, PR, NSRC>), dim3((unsigned)nblk),
+  hipLaunchKernelGGL((k_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC>), dim3((unsigned)nblk),
                      dim3(tile_threads<NTL, 0, PR>()), 0, s, a);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }

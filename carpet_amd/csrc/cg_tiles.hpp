@@ -52,14 +52,18 @@ __device__ __forceinline__ int xcd_remap(int b, int n) {
   return xcd * per + min(xcd, rem) + slot;
 }
 
-// LDS footprint (doubles) of one tensor tile; XQ = bases per thread in the
-// x-pass (2: rows padded to an even stride for 16-byte LDS accesses); NB =
-// buffers of the window and of the x-pass results (2 for the pipelined
+// LDS footprint (doubles) of one tensor tile; window rows are padded to an
+// even stride for the x-pass's 16-byte LDS accesses; NB = buffers of the window and of the x-pass results (2 for the pipelined
 // schedule)
-template <class L, int NTL, int CX, int CY, int XQ = 1, int NB = 1> struct TensorLds {
+template <class L, int NTL, int CX, int CY, int NB = 1> struct TensorLds {
   static constexpr int SPAN = L::TMAXALL - L::TMINALL;
-  static constexpr int WX = CX + SPAN;
-  static constexpr int WXS = XQ == 1 ? WX : (WX + 1) / 2 * 2;
+  // window columns: the taps of CX bases, and of the first child of the base
+  // after them (a tile whose first column is a second child ends with it)
+  static constexpr int T0 = L::TMIN[0] - L::TMINALL + L::NTAP[0]; // end of a first child's taps
+  static constexpr int WX = CX + (SPAN > T0 ? SPAN : T0);
+  // pairs of window columns that the four children of two bases reach
+  static constexpr int NP = ((SPAN > T0 ? SPAN : T0) + 3) / 2;
+  static constexpr int WXS = (CX - 2 + 2 * NP > WX ? CX - 2 + 2 * NP : WX + 1) / 2 * 2;
   static constexpr int WY = CY + SPAN;
   static constexpr int A = NTL * WY * WXS; // one window buffer
   static constexpr int X = NTL * WY * 2 * CX; // one x-pass buffer
@@ -128,8 +132,7 @@ template <int I, int N, class F> __device__ __forceinline__ bool unroll_while(F 
 
 // One z-marching tile; tile b indexes (x tile, y tile, z chunk) of a.
 // PR: precision mode (Prec); PF: planes loaded ahead of their use (register
-// buffers per plane); XQ: coarse bases per thread in the x-pass (1, or 2 with
-// paired LDS accesses); PIPE: schedule of the plane loop (0: window store,
+// buffers per plane); PIPE: schedule of the plane loop (0: window store,
 // barrier, x-pass, barrier, y-pass per plane; 1: software pipeline -- the
 // window of plane c, the x-pass of plane c-1 and the y-pass of plane c-2
 // between two barriers, with double-buffered window and x-pass results);
@@ -137,9 +140,9 @@ template <int I, int N, class F> __device__ __forceinline__ bool unroll_while(F 
 // the window is stored (time interpolation before the spatial stencil, exact
 // by linearity up to rounding; the FP32-storage, FP64-arithmetic mode), so
 // the passes run once instead of once per level.
-// smem must be 16-byte aligned and hold TensorLds<..., XQ, PIPE ? 2 : 1>
-template <class L, int NTL, int CX, int CY, int IPT, int PR = 0, int PF = 1, int XQ = 1,
-          int PIPE = 0, int NSRC = NTL>
+// smem must be 16-byte aligned and hold TensorLds<..., PIPE ? 2 : 1>
+template <class L, int NTL, int CX, int CY, int IPT, int PR = 0, int PF = 1, int PIPE = 0,
+          int NSRC = NTL>
 __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *smem) {
   using TS = typename Prec<PR>::S; // storage
   using CT = typename Prec<PR>::C; // arithmetic of the passes
@@ -150,9 +153,9 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
   constexpr int NT = FX * CY / IPT;
   constexpr int NQY = NT / FX;
   static_assert(NQY * IPT == CY, "tile rows must divide among threads");
-  static_assert(XQ == 1 || (XQ == 2 && CX % 2 == 0), "x-pass bases per thread: 1 or 2");
+  static_assert(CX % 2 == 0, "the x-pass takes two bases per thread");
   constexpr int NB = PIPE ? 2 : 1;
-  using LD = TensorLds<L, NTL, CX, CY, XQ, NB>;
+  using LD = TensorLds<L, NTL, CX, CY, NB>;
   constexpr int WX = LD::WX;
   constexpr int WXS = LD::WXS; // LDS row stride of the window
   constexpr int WY = LD::WY;
@@ -180,7 +183,11 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
   const int ty = b % a.ntiles[1];
   const int tz = b / a.ntiles[1];
 
-  const int qx0 = a.qlo[0] + tx * CX;
+  // tile column j is fine point f0 + j: the child (f0 + j) & 1 of base
+  // (f0 + j) >> 1; odd: a tile starts with a second child
+  const int f0 = a.off[0] - a.sx + tx * FX;
+  const int qx0 = f0 >> 1;
+  const bool odd = f0 & 1;
   const int qy0 = a.qlo[1] + ty * CY;
   const int qz0 = a.qlo[2] + tz * a.zchunk;
   const int qz1 = min(qz0 + a.zchunk, a.qlo[2] + a.nq[2]) - 1;
@@ -193,7 +200,7 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
 
   const int tid = threadIdx.x;
   const int fx = tid % FX, qyl = tid / FX;
-  const int gfx = 2 * qx0 + fx - a.off[0];
+  const int gfx = tx * FX + fx - a.sx;
   const bool xin = gfx >= 0 && gfx < a.n[0];
 
   // this thread's share of the plane window: offsets into the source plane
@@ -265,43 +272,37 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
   auto xpass = [&](auto Bc) {
     auto A = Abuf(decltype(Bc)::value);
     auto X = Xbuf(decltype(Bc)::value);
-    // work items (time level, row, base group) spread over all threads
-    if constexpr (XQ == 1) {
-      for (int e = tid; e < NTL * WY * CX; e += NT) {
-        const int tl = e / (WY * CX), e2 = e - tl * (WY * CX);
-        const int r = e2 / CX, q = e2 - r * CX;
-        const WT *w = &A[tl][r][q - L::TMINALL];
-        const CT v0 = line_apply<L, 0, CT>([&](int t) { return w[L::TMIN[0] + t]; });
-        const CT v1 = line_apply<L, 1, CT>([&](int t) { return w[L::TMIN[1] + t]; });
-        X[tl][r][2 * q] = v0;
-        X[tl][r][2 * q + 1] = v1;
-      }
-    } else {
-      // bases q0, q0+1 from the window columns q0 .. q0+SPAN+1 (window
-      // column 0 is offset TMINALL of base 0), read and written in pairs
-      using P2 = typename Pair<WT>::T;
-      using C2 = typename Pair<CT>::T;
-      constexpr int NP = (LD::SPAN + 3) / 2;
-      constexpr int NQ2 = WY * (CX / 2);
-      for (int e = tid; e < NTL * NQ2; e += NT) {
-        const int tl = e / NQ2, e2 = e - tl * NQ2;
-        const int r = e2 / (CX / 2), q0 = 2 * (e2 - r * (CX / 2));
-        WT v[2 * NP];
+    // work items (time level, row, base pair) spread over all threads: bases
+    // q0, q0+1 from the window columns q0 .. (window column 0 is offset
+    // TMINALL of base 0), read and written in pairs
+    using P2 = typename Pair<WT>::T;
+    using C2 = typename Pair<CT>::T;
+    constexpr int NP = LD::NP;
+    constexpr int NQ2 = WY * (CX / 2);
+    for (int e = tid; e < NTL * NQ2; e += NT) {
+      const int tl = e / NQ2, e2 = e - tl * NQ2;
+      const int r = e2 / (CX / 2), q0 = 2 * (e2 - r * (CX / 2));
+      WT v[2 * NP];
 #pragma unroll
-        for (int m = 0; m < NP; ++m) {
-          const P2 p = *reinterpret_cast<const P2 *>(&A[tl][r][q0 + 2 * m]);
-          v[2 * m] = p.x;
-          v[2 * m + 1] = p.y;
-        }
-        constexpr int O0 = L::TMIN[0] - L::TMINALL, O1 = L::TMIN[1] - L::TMINALL;
-        C2 lo, hi;
-        lo.x = line_apply<L, 0, CT>([&](int t) { return v[O0 + t]; });
-        lo.y = line_apply<L, 1, CT>([&](int t) { return v[O1 + t]; });
-        hi.x = line_apply<L, 0, CT>([&](int t) { return v[1 + O0 + t]; });
-        hi.y = line_apply<L, 1, CT>([&](int t) { return v[1 + O1 + t]; });
-        *reinterpret_cast<C2 *>(&X[tl][r][2 * q0]) = lo;
-        *reinterpret_cast<C2 *>(&X[tl][r][2 * q0 + 2]) = hi;
+      for (int m = 0; m < NP; ++m) {
+        const P2 p = *reinterpret_cast<const P2 *>(&A[tl][r][q0 + 2 * m]);
+        v[2 * m] = p.x;
+        v[2 * m + 1] = p.y;
       }
+      constexpr int O0 = L::TMIN[0] - L::TMINALL, O1 = L::TMIN[1] - L::TMINALL;
+      const CT b = line_apply<L, 1, CT>([&](int t) { return v[O1 + t]; });
+      const CT c = line_apply<L, 0, CT>([&](int t) { return v[1 + O0 + t]; });
+      const CT d = line_apply<L, 1, CT>([&](int t) { return v[1 + O1 + t]; });
+      C2 lo, hi;
+      if (odd) {
+        lo.x = b, lo.y = c, hi.x = d;
+        hi.y = line_apply<L, 0, CT>([&](int t) { return v[2 + O0 + t]; });
+      } else {
+        lo.x = line_apply<L, 0, CT>([&](int t) { return v[O0 + t]; });
+        lo.y = b, hi.x = c, hi.y = d;
+      }
+      *reinterpret_cast<C2 *>(&X[tl][r][2 * q0]) = lo;
+      *reinterpret_cast<C2 *>(&X[tl][r][2 * q0 + 2]) = hi;
     }
   };
   // y-pass of plane p (x buffer B) into ring slot J, then the z-emission of
@@ -820,8 +821,6 @@ __device__ __forceinline__ void tvd_cell(const PointArgs &a, int qx, int qy, int
 // threads.  With 2-3 time levels the register ring is 2-3x larger, so each
 // thread keeps one base row (IPT 1, 512 threads); 8 base rows per tile cut
 // the y halo of the x-pass and of the window loads to (8+span)/8.
-// XQ = 2: the x-pass reads and writes LDS in 16-byte pairs (two bases per
-// thread), a third fewer LDS reads than one base per thread.
 // SH = 0 ("wide", 32 x 8 bases) suits large regions; SH = 1 ("narrow",
 // 16 x 16 bases) wastes fewer lanes on regions of a few dozen points per
 // axis and has a smaller x halo per fine point.  PR: precision mode; the
@@ -830,45 +829,45 @@ __device__ __forceinline__ void tvd_cell(const PointArgs &a, int qx, int qy, int
 // half as large per point.
 template <int NTL, int SH = 0, int PR = 0> struct TileShape : TileShape<NTL, SH, 0> {};
 template <> struct TileShape<1, 0, 0> {
-  static constexpr int CX = 32, CY = 8, IPT = 2, XQ = 2;
+  static constexpr int CX = 32, CY = 8, IPT = 2;
 };
 template <> struct TileShape<2, 0, 0> {
-  static constexpr int CX = 32, CY = 8, IPT = 1, XQ = 2;
+  static constexpr int CX = 32, CY = 8, IPT = 1;
 };
 template <> struct TileShape<3, 0, 0> {
-  static constexpr int CX = 32, CY = 8, IPT = 1, XQ = 2;
+  static constexpr int CX = 32, CY = 8, IPT = 1;
 };
 template <> struct TileShape<1, 1, 0> {
-  static constexpr int CX = 16, CY = 16, IPT = 2, XQ = 2;
+  static constexpr int CX = 16, CY = 16, IPT = 2;
 };
 template <> struct TileShape<2, 1, 0> {
-  static constexpr int CX = 16, CY = 16, IPT = 1, XQ = 2;
+  static constexpr int CX = 16, CY = 16, IPT = 1;
 };
 template <> struct TileShape<3, 1, 0> {
-  static constexpr int CX = 16, CY = 16, IPT = 1, XQ = 2;
+  static constexpr int CX = 16, CY = 16, IPT = 1;
 };
 template <> struct TileShape<1, 0, 1> {
-  static constexpr int CX = 64, CY = 8, IPT = 2, XQ = 2;
+  static constexpr int CX = 64, CY = 8, IPT = 2;
 };
 // small tiles (FP64 batch only) for regions a few fine points across in x
 // and in y or z: edges and corners of ghost and buffer shells, faces thin
 // in x, where a 32x8 or 16x16 tile keeps a tenth of its lanes busy or less
 template <int NTL> struct TileShape<NTL, 2, 0> {
-  static constexpr int CX = 8, CY = 8, IPT = 1, XQ = 2;
+  static constexpr int CX = 8, CY = 8, IPT = 1;
 };
 // slim tiles (FP64 batch only), 4 x 16 bases, for regions a few fine points
 // across in x and long in y: ghost and buffer faces normal to x, where an
 // 8x8 tile leaves most of its x lanes and window columns idle
 template <int NTL> struct TileShape<NTL, 3, 0> {
-  static constexpr int CX = 4, CY = 16, IPT = 1, XQ = 2;
+  static constexpr int CX = 4, CY = 16, IPT = 1;
 };
 // the pipelined schedule (double-buffered window and x-pass results) where
 // its LDS fits the 64 KB of a static allocation, else two barriers per plane
-template <class L, int NTL, int CX, int CY, int XQ> constexpr int pipe_fits() {
-  return TensorLds<L, NTL, CX, CY, XQ, 2>::TOTAL * 8 <= 65536 ? 1 : 0;
+template <class L, int NTL, int CX, int CY> constexpr int pipe_fits() {
+  return TensorLds<L, NTL, CX, CY, 2>::TOTAL * 8 <= 65536 ? 1 : 0;
 }
-template <class L, int NTL, int CX, int CY, int XQ> constexpr int tile_lds() {
-  return TensorLds<L, NTL, CX, CY, XQ, pipe_fits<L, NTL, CX, CY, XQ>() ? 2 : 1>::TOTAL;
+template <class L, int NTL, int CX, int CY> constexpr int tile_lds() {
+  return TensorLds<L, NTL, CX, CY, pipe_fits<L, NTL, CX, CY>() ? 2 : 1>::TOTAL;
 }
 
 // time levels the tile passes carry: the FP32-storage, FP64-arithmetic mode

@@ -64,6 +64,7 @@ constexpr int PT_DEFAULT = 4096;
 constexpr int ZCHUNK_DEFAULT = 16;
 
 
+
 // points per thread and round of the pointwise kernel: items of 256, 512,
 // 1024 points take one round of 1, 2, 4 points per thread, larger items
 // rounds of 8 (a plain copy streams fastest with one point per thread and
@@ -593,7 +594,8 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     // levels 1.35 against 1.38 ms; 8 x 384^3 with FP32 storage 633 against
     // 642 us; 8 x 320^3 cell ENO<3> equal; 5 x 256^3 vertex ENO, 3 levels,
     // 378 against 323 us; 8 x 231x165x297 order 3, 2 levels, 240 against
-    // 216 us.)
+    // 216 us.)  Regions of 2^20 points and up whose items fit one round of
+    // resident workgroups are persistent too, without counters (one_round).
     l.wpc = g.is_tensor && !g.small && median_pts >= (1LL << 25) ? 0 : -1;
     // tile shape: the class's (its regions were routed by shape)
     l.shape = !g.is_tensor ? 0 : g.small ? g.small : g.bigsh;
@@ -645,7 +647,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
       if (tile_cfg < 0 && !(tuned && tuned->count(l.key))) {
         const int span = line_span(g.kind, g.order);
         std::vector<double> mk;
-        const int zcs[5] = {128, 64, 32, 16, 8};
+        const int zcs[6] = {128, 64, 32, 16, 8, 4};
         for (int zc : zcs) {
           std::priority_queue<double, std::vector<double>, std::greater<double>> q;
           for (int w = 0; w < full_grid; ++w)
@@ -672,7 +674,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
         // against 1.74 ms at 128)
         const int first = fp64_only(g.kind) ? 1 : 0;
         const double best = *std::min_element(mk.begin() + first, mk.end());
-        for (int i = first; i < 5; ++i)
+        for (int i = first; i < 6; ++i)
           if (mk[i] <= 1.03 * best) {
             l.zchunk = zcs[i];
             break;
@@ -780,7 +782,12 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     }
     l.item_off = append(items.data(), items.size() * sizeof(Item));
     l.counter = (int)dev.launches.size();
-    if (l.wpc == -1) {
+    if (l.wpc == -1 && !(tuned && tuned->count(l.key)) && g.is_tensor && !g.small &&
+        median_pts >= (1LL << 20) && l.nitems <= full_grid)
+      l.wpc = 0;
+    // a persistent grid that holds every item at once needs no counters
+    l.one_round = l.wpc >= 0 && g.is_tensor && l.nitems <= full_grid;
+    if (l.wpc == -1 || l.one_round) {
       // grid mode: 8 x the longest segment (in groups of ni items)
       long long longest = 1;
       for (int x = 0; x < 8; ++x)
@@ -890,7 +897,7 @@ int batch_device_run(BatchDevice &dev, hipStream_t st) {
   // only persistent launches use the work counters
   bool persistent = false;
   for (const BatchLaunch &l : dev.launches)
-    persistent = persistent || l.wpc >= 0;
+    persistent = persistent || (l.wpc >= 0 && !l.one_round);
   if (persistent)
     hipLaunchKernelGGL(k_zero_counters, dim3((8 * dev.ncounters + 255) / 256), dim3(256), 0, st,
                        dev.counters, 8 * dev.ncounters);

@@ -65,7 +65,7 @@ int batch_tensor_go(const BatchLaunch &l, const TensorArgs *td, const Item *item
   constexpr int NTL = pass_levels(NSRC, PR);
   using T = TileShape<NTL, SH, PR>;
   const dim3 block(tile_threads<NTL, SH, PR>());
-  if (l.wpc == -1)
+  if (l.wpc == -1 || l.one_round)
     hipLaunchKernelGGL((k_grid_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC>), dim3(l.grid), block,
                        0, st, td, items, seg);
   else

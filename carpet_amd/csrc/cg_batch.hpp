@@ -38,8 +38,10 @@ struct BatchLaunch {
   std::string key; // tuner cache key (class + box-size histogram bucket)
   std::vector<int> members; // transfer indices in descriptor order
   size_t desc_bytes;        // bytes of the descriptor array
-  std::vector<int> sx;      // tensor: each descriptor's tile grid shift, which the items were cut
-                            // with (kept when new storage has another alignment)
+  // each descriptor's tile grid shift (tensor) or row slots (pointwise),
+  // which the items were cut with (kept when new storage has another
+  // alignment)
+  std::vector<int> sx, nxp;
 };
 
 // one work item: a tile (tensor) or a run of points (pointwise) of one

@@ -125,7 +125,7 @@ __device__ __forceinline__ void point_item(const PointArgs &a, unsigned tile, in
     else
       tvd_item<3>(a, tile, pt);
   } else {
-    const unsigned nx = (unsigned)a.n[0];
+    const unsigned nx = (unsigned)a.nxp;
     const unsigned nxy = nx * (unsigned)a.n[1];
     const unsigned tot = nxy * (unsigned)a.n[2]; // < 2^31 (checked on the host)
     const unsigned e0 = tile * (unsigned)pt;
@@ -143,9 +143,11 @@ __device__ __forceinline__ void point_item(const PointArgs &a, unsigned tile, in
           const unsigned k = fastdiv(e, a.fxy);
           const unsigned r = e - k * nxy;
           const unsigned j = fastdiv(r, a.fx);
-          const unsigned i = r - j * nx;
-          v[u] = point_value<OP>(a, (int)i, (int)j, (int)k);
-          o[u] = (long long)i + a.dj * j + a.dk * k;
+          const int i = (int)(r - j * nx) - a.sx;
+          if (i >= 0 && i < a.n[0]) {
+            v[u] = point_value<OP>(a, i, (int)j, (int)k);
+            o[u] = i + a.dj * j + a.dk * k;
+          }
         }
       }
 #pragma unroll
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(256) void k_grid_point_n(const PointArgs *__restric
     if (it < i1) {
       const Item w = items[it];
       const PointArgs &a = descs[w.desc];
-      const unsigned nx = (unsigned)a.n[0];
+      const unsigned nx = (unsigned)a.nxp;
       const unsigned nxy = nx * (unsigned)a.n[1];
       const unsigned tot = nxy * (unsigned)a.n[2];
       const unsigned e = w.tile * 256u + threadIdx.x;
@@ -211,9 +213,11 @@ __global__ __launch_bounds__(256) void k_grid_point_n(const PointArgs *__restric
         const unsigned k = fastdiv(e, a.fxy);
         const unsigned r = e - k * nxy;
         const unsigned j = fastdiv(r, a.fx);
-        const unsigned i = r - j * nx;
-        v[u] = point_value<OP>(a, (int)i, (int)j, (int)k);
-        q[u] = (gdst_t)a.dst + ((long long)i + a.dj * j + a.dk * k);
+        const int i = (int)(r - j * nx) - a.sx;
+        if (i >= 0 && i < a.n[0]) {
+          v[u] = point_value<OP>(a, i, (int)j, (int)k);
+          q[u] = (gdst_t)a.dst + (i + a.dj * j + a.dk * k);
+        }
       }
     }
   }
@@ -314,16 +318,27 @@ TensorArgs tensor_desc(const BatchLaunch &l, const Transfer &t, int sx = -1) {
   return a;
 }
 
-PointArgs point_desc(const BatchLaunch &l, const Transfer &t) {
+// work units of a pointwise transfer per axis: row slots, or TVD's coarse
+// parent cells
+void point_units(const BatchLaunch &l, const PointArgs &a, long long *u) {
+  for (int d = 0; d < 3; ++d)
+    u[d] = l.op == PO_TVD ? ((a.off[d] + a.n[d] - 1) >> 1) - (a.off[d] >> 1) + 1 : d == 0 ? a.nxp : a.n[d];
+}
+
+// nxp > 0: the row slots that the transfer's items were cut with
+PointArgs point_desc(const BatchLaunch &l, const Transfer &t, int sx = 0, int nxp = 0) {
   PointArgs a = t.is_prolong ? t.pr.p : t.pt.a;
   if (l.op == PO_INTERP && !t.is_prolong && t.pt.op == PO_COPY) {
     a.ntl = 1;
     a.s[0] = 1.0;
   }
-  // work units: destination points, or TVD's coarse parent cells
+  point_rows(a);
+  if (nxp > 0) {
+    a.sx = sx;
+    a.nxp = nxp;
+  }
   long long u[3];
-  for (int d = 0; d < 3; ++d)
-    u[d] = l.op == PO_TVD ? ((a.off[d] + a.n[d] - 1) >> 1) - (a.off[d] >> 1) + 1 : a.n[d];
+  point_units(l, a, u);
   a.fx = make_fastdiv((unsigned)u[0]);
   a.fxy = make_fastdiv((unsigned)(u[0] * u[1]));
   return a;
@@ -458,7 +473,7 @@ void batch_launch_descs(const BatchLaunch &l, const std::vector<Transfer> &tr, c
       const TensorArgs a = tensor_desc(l, t, l.sx[i]);
       std::memcpy(out + i * sizeof(TensorArgs), &a, sizeof a);
     } else {
-      const PointArgs a = point_desc(l, t);
+      const PointArgs a = point_desc(l, t, l.sx[i], l.nxp[i]);
       std::memcpy(out + i * sizeof(PointArgs), &a, sizeof a);
     }
   }
@@ -582,10 +597,13 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     // restriction of the same set: 0.77 ms against 0.81 ms with 4096)
     else if (g.op == PO_TVD || g.op == PO_RESTRICT_CC || g.op == PO_RESTRICT_CC_O3 || g.op == PO_RESTRICT_CC_O5)
       l.pt = 1024;
-    // copies: 2048 points (2000 regions of 8-96 points per axis: 19.03 ms
-    // per step against 19.43 ms with 4096)
+    // copies 1024 slots, injections 512 (2000 regions of 8-96 points per
+    // axis x 4, at 512, 1024, 2048 and 4096: copies 1.53, 1.29, 1.45 and
+    // 1.53 ms, injections 0.279, 0.304, 0.311 and 0.317 ms)
     else if (g.op == PO_COPY)
-      l.pt = 2048;
+      l.pt = 1024;
+    else if (g.op == PO_RESTRICT_VC)
+      l.pt = 512;
     // tensor tiles of very large regions (median 2^25 points and up):
     // persistent grid (its workgroups take the tiles in order, so
     // neighbouring tiles march through z together and share halo rows in
@@ -703,15 +721,15 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
       std::vector<PointArgs> descs;
       for (int m : members) {
         const PointArgs a = point_desc(l, tr[m]);
-        // work units: destination points, or TVD's coarse parent cells
         long long u[3];
-        for (int d = 0; d < 3; ++d)
-          u[d] = g.op == PO_TVD ? ((a.off[d] + a.n[d] - 1) >> 1) - (a.off[d] >> 1) + 1 : a.n[d];
+        point_units(l, a, u);
         const long long tot = u[0] * u[1] * u[2];
         if (tot >= (1LL << 31) - l.pt)
           return set_error(CG_ERR_ARG, "region too large for the batch");
         const unsigned d = (unsigned)descs.size();
         descs.push_back(a);
+        l.sx.push_back(a.sx);
+        l.nxp.push_back(a.nxp);
         first.push_back((int)items.size());
         const long long nt = (tot + l.pt - 1) / l.pt;
         for (long long t = 0; t < nt; ++t) {

@@ -92,7 +92,9 @@ struct PointArgs {
   int stag;             // staggered operators: bit d set = staggered in direction d;
                         // restrict_3d_vc_rf2: bit d set = direction d cell-centred
   int sorder;           //   prolongation order (2 or 3)
-  FastDiv fx, fxy;      // division by n[0] and n[0]*n[1] (batch work items)
+  int nxp, sx;          // a row is walked in nxp slots, its point i in slot i + sx
+                        // (point_rows; TVD: coarse parents, not slots)
+  FastDiv fx, fxy;      // division by nxp and nxp*n[1] (TVD: by the parents)
 };
 
 // tile configuration of the tensor kernel
@@ -119,6 +121,8 @@ inline int tiles_x(const TensorArgs &a, int cx, int sx) { return (a.n[0] + sx + 
 // computes ntiles/zchunk (and sx, unless it is set) of a for a tile
 // configuration; returns block count
 long long tensor_tiles(TensorArgs &a, const TileCfg &cfg);
+// chooses the slots of a's rows (nxp, sx) and sets fx, fxy
+void point_rows(PointArgs &a);
 int launch_point(int op, const PointArgs &a, hipStream_t s);
 int launch_fill(double *dst, double v, size_t n, hipStream_t s);
 int launch_stream_copy(double *dst, const double *src, size_t n, hipStream_t s);

@@ -1,6 +1,7 @@
-"""Tensor tiles start at a 128-byte line of the destination rows: regions at
-every offset from a line, of widths around the tiles' and of both parities,
-per call and batched, equal the oracle bit for bit."""
+"""Tensor tiles and the rows of pointwise operators start at a 128-byte line of
+the destination: regions at every offset from a line, of widths around the
+tiles' and lines' and of both parities, per call and batched, equal the oracle
+bit for bit."""
 import numpy as np
 import pytest
 
@@ -64,6 +65,69 @@ def test_offsets_match_oracle(cent, op, order, ntl, ny, nz):
             if not same(got, ref[k]):
                 raise AssertionError(f"{how}: {k} differs {first_diff(got, ref[k])}")
         if how == "batched":
+            b.close()
+        w.free(dev)
+
+
+def _point_regions(what, ny, nz):
+    """As _regions, for copies, injections and cell restrictions, and a same-
+    level time interpolation."""
+    w = Workload(what)
+    s, cent = {"copy": (1, V), "interp": (1, V), "inject": (2, V), "average": (4, C)}[what]
+    lo = 4 if cent == V else 2
+    srcs = ["a", "b"] if what == "interp" else ["a"]
+    f = s if what in ("copy", "interp") else s // 2
+    for i, nm in enumerate(srcs):
+        if what in ("copy", "interp"):
+            sbox = Box((lo - 3,) * 3, (lo + 190, lo + 60, lo + 40), (1,) * 3)
+        elif cent == V:
+            sbox = Box((0,) * 3, (360, 110, 70), (f,) * 3)
+        else:
+            sbox = Box((1,) * 3, (1 + 2 * 360, 1 + 2 * 110, 1 + 2 * 70), (f,) * 3)
+        w.arrays[nm] = ArraySpec(sbox, seed=60 + i)
+    for i, n in enumerate((1, 3, 7, 8, 15, 16, 17, 31, 33, 64, 65, 100, 130)):
+        for k in ((i * 7) % 16, (i * 5 + 1) % 16, 17):
+            own = Box((lo, lo, lo), (lo + 150 * s, lo + 45 * s, lo + 30 * s), (s,) * 3)
+            reg = Box((lo + k * s, lo + s, lo), (lo + (k + n - 1) * s, lo + ny * s, lo + (nz - 1) * s), (s,) * 3)
+            nm = f"d{n}_{k}"
+            w.arrays[nm] = ArraySpec(own.expand((2, 1, 1), (2, 1, 1)), owned=own, seed=300 + 31 * n + k)
+            t = ([0.0, -1.0], -0.25) if what == "interp" else ([0.0], 0.0)
+            w.steps.append(Transfer(nm, nm, srcs, t[0], reg, reg, t[1], cg.OP_LAGRANGE, cent, 1, len(srcs) - 1, phase=0))
+            w.outputs.append(nm)
+    return w
+
+
+@pytest.mark.parametrize("ny,nz", [(40, 20), (3, 3), (1, 1)])
+@pytest.mark.parametrize("what", ["copy", "interp", "inject", "average"])
+def test_point_offsets_match_oracle(what, ny, nz):
+    w = _point_regions(what, ny, nz)
+    ref = run_oracle(w)
+    st = cg.Stream()
+    for how in ("per call", "batched", "moved"):
+        dev = w.allocate()
+        keep = []
+        if how == "per call":
+            w.run_steps(dev, st)
+        else:
+            b = w.batch(dev)
+            b.finalize()
+            if how == "moved":  # storage whose rows start elsewhere in a line
+                for k in w.outputs:
+                    a = dev[k]
+                    n = int(np.prod(a.padext))
+                    keep.append((a, cg.DeviceArray(Box((0, 0, 0), (n + 31, 0, 0), (1, 1, 1)), padext=(n + 32, 1, 1))))
+                    m = cg.DeviceArray.view(a.box, keep[-1][1].ptr + 8 * 5, a.padext)
+                    m.fill(np.nan, stream=st)
+                    m.fill_hash(w.arrays[k].seed, stream=st)
+                    b.set_storage([(a, m)])
+                    dev[k] = m
+            b.run(st)
+        st.synchronize()
+        for k in ref:
+            got = dev[k].download()
+            if not same(got, ref[k]):
+                raise AssertionError(f"{how}: {k} differs {first_diff(got, ref[k])}")
+        if how != "per call":
             b.close()
         w.free(dev)
 

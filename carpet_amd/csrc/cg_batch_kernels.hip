@@ -138,16 +138,14 @@ __device__ __forceinline__ void point_item(const PointArgs &a, unsigned tile, in
 #pragma unroll
       for (int u = 0; u < PU; ++u) {
         const unsigned e = eb + u * 256u + threadIdx.x;
+        const unsigned k = fastdiv(e, a.fxy);
+        const unsigned r = e - k * nxy;
+        const unsigned j = fastdiv(r, a.fx);
+        const int i = (int)(r - j * nx) - a.sx;
         o[u] = -1;
-        if (e < e1) {
-          const unsigned k = fastdiv(e, a.fxy);
-          const unsigned r = e - k * nxy;
-          const unsigned j = fastdiv(r, a.fx);
-          const int i = (int)(r - j * nx) - a.sx;
-          if (i >= 0 && i < a.n[0]) {
-            v[u] = point_value<OP>(a, i, (int)j, (int)k);
-            o[u] = i + a.dj * j + a.dk * k;
-          }
+        if (e < e1 && i >= 0 && i < a.n[0]) {
+          v[u] = point_value<OP>(a, i, (int)j, (int)k);
+          o[u] = i + a.dj * j + a.dk * k;
         }
       }
 #pragma unroll
@@ -209,15 +207,13 @@ __global__ __launch_bounds__(256) void k_grid_point_n(const PointArgs *__restric
       const unsigned nxy = nx * (unsigned)a.n[1];
       const unsigned tot = nxy * (unsigned)a.n[2];
       const unsigned e = w.tile * 256u + threadIdx.x;
-      if (e < tot) {
-        const unsigned k = fastdiv(e, a.fxy);
-        const unsigned r = e - k * nxy;
-        const unsigned j = fastdiv(r, a.fx);
-        const int i = (int)(r - j * nx) - a.sx;
-        if (i >= 0 && i < a.n[0]) {
-          v[u] = point_value<OP>(a, i, (int)j, (int)k);
-          q[u] = (gdst_t)a.dst + (i + a.dj * j + a.dk * k);
-        }
+      const unsigned k = fastdiv(e, a.fxy);
+      const unsigned r = e - k * nxy;
+      const unsigned j = fastdiv(r, a.fx);
+      const int i = (int)(r - j * nx) - a.sx;
+      if (e < tot && i >= 0 && i < a.n[0]) {
+        v[u] = point_value<OP>(a, i, (int)j, (int)k);
+        q[u] = (gdst_t)a.dst + (i + a.dj * j + a.dk * k);
       }
     }
   }
@@ -262,7 +258,7 @@ struct Group {
 double tile_busy(const TensorArgs &a, int ntl, int prec, int span, int sh) {
   int cx, cy, th;
   tile_shape(ntl, prec, &cx, &cy, &th, sh);
-  return (double)tiles_x(a, cx, tile_shift(a, cx, prec ? 4 : 8)) * ((a.nq[1] + cy - 1) / cy) * (a.nq[2] + span) * cx *
+  return (double)tiles_x(a, cx, tile_shift(a, cx, prec ? 4 : 8)) * tiles_y(a, cy) * (a.nq[2] + span) * cx *
          (cy + span);
 }
 
@@ -591,12 +587,16 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
       l.ni = CG_POINT_NI;
     }
     // TVD items count coarse parent cells (8 fine points each): 1024 cells
-    // (measured on 8 variables of 192^3 -> 384^3: 0.98 ms against 1.05 ms
-    // with 4096 and 1.11 ms with 256); cell-centred restriction (8 or more
-    // children per point) likewise 1024 points (the 384^3 -> 192^3
-    // restriction of the same set: 0.77 ms against 0.81 ms with 4096)
-    else if (g.op == PO_TVD || g.op == PO_RESTRICT_CC || g.op == PO_RESTRICT_CC_O3 || g.op == PO_RESTRICT_CC_O5)
+    // (8 variables of 192^3 -> 384^3: 0.98 ms against 1.00 ms with 512, 1.01
+    // with 2048 and 1.10 with 256); higher-order cell restrictions 1024
+    // points
+    else if (g.op == PO_TVD || g.op == PO_RESTRICT_CC_O3 || g.op == PO_RESTRICT_CC_O5)
       l.pt = 1024;
+    // cell-centred restriction (8 children per point): 256 (the 384^3 ->
+    // 192^3 restriction of the same set, at 256, 512, 1024 and 4096: 0.70,
+    // 0.74, 0.76 and 0.79 ms)
+    else if (g.op == PO_RESTRICT_CC)
+      l.pt = 256;
     // copies 1024 slots, injections 512 (2000 regions of 8-96 points per
     // axis x 4, at 512, 1024, 2048 and 4096: copies 1.53, 1.29, 1.45 and
     // 1.53 ms, injections 0.279, 0.304, 0.311 and 0.317 ms)
@@ -673,7 +673,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
           for (int m : members) {
             const TensorArgs &a = tr[m].pr.t;
             const long long nxy =
-                (long long)tiles_x(a, cfg.cx, tile_shift(a, cfg.cx, g.prec ? 4 : 8)) * ((a.nq[1] + cfg.cy - 1) / cfg.cy);
+                (long long)tiles_x(a, cfg.cx, tile_shift(a, cfg.cx, g.prec ? 4 : 8)) * tiles_y(a, cfg.cy);
             for (int z0 = 0; z0 < a.nq[2]; z0 += zc)
               for (long long t = 0; t < nxy; ++t) {
                 const double at = q.top();

@@ -28,7 +28,7 @@ long long tensor_tiles(TensorArgs &a, const TileCfg &cfg) {
   if (a.sx < 0)
     a.sx = tile_shift(a, cfg.cx, cfg.es);
   a.ntiles[0] = tiles_x(a, cfg.cx, a.sx);
-  a.ntiles[1] = (a.nq[1] + cfg.cy - 1) / cfg.cy;
+  a.ntiles[1] = tiles_y(a, cfg.cy);
   a.zchunk = cfg.zchunk > 0 ? cfg.zchunk : a.nq[2];
   a.ntiles[2] = (a.nq[2] + a.zchunk - 1) / a.zchunk;
   return (long long)a.ntiles[0] * a.ntiles[1] * a.ntiles[2];

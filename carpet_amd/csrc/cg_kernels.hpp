@@ -40,6 +40,8 @@ struct TensorArgs {
   int ntiles[3];      // tile counts: x, y (in CX/CY bases), z (chunks)
   int sx;             // the tile grid starts sx fine columns before the region
                       // (tensor_tiles; < 0: not chosen yet)
+  int sy;             // and sy (0 or 1) fine rows: tile rows pair up as the
+                      // kind's children do
   int zchunk;         // coarse bases per z chunk
   double s[3];        // time weights
   double s2[2];       // ENO time rule: weights of the fallback pair
@@ -118,6 +120,7 @@ int launch_tensor(int kind, int order, int ntl, int prec, const TensorArgs &a,
 // and the tiles along x that follow from it
 int tile_shift(const TensorArgs &a, int cx, int es);
 inline int tiles_x(const TensorArgs &a, int cx, int sx) { return (a.n[0] + sx + 2 * cx - 1) / (2 * cx); }
+inline int tiles_y(const TensorArgs &a, int cy) { return (a.n[1] + a.sy + 2 * cy - 1) / (2 * cy); }
 // computes ntiles/zchunk (and sx, unless it is set) of a for a tile
 // configuration; returns block count
 long long tensor_tiles(TensorArgs &a, const TileCfg &cfg);

@@ -356,6 +356,7 @@ int plan_prolong(int kind, int order, const Arr &src, const void *const *srcs,
     t.s[l] = l < ntl ? s[l] : 0.0;
   t.nlev = ntl;
   t.sx = -1;
+  t.sy = (t.off[1] & 1) ^ (kind == PK_ENO ? 1 : 0);
   if (eno && ntl == 3) {
     t.teno = 1;
     t.l0 = eno->l0;
@@ -391,7 +392,7 @@ int launch_prolong(const ProlongPlan &pl, int prec, hipStream_t st) {
     int threads = 0;
     tile_shape(pl.ntl, prec, &cfg.cx, &cfg.cy, &threads);
     const long long cols = (long long)tiles_x(a, cfg.cx, tile_shift(a, cfg.cx, cfg.es)) *
-                           ((a.nq[1] + cfg.cy - 1) / cfg.cy);
+                           tiles_y(a, cfg.cy);
     int zc = std::min(a.nq[2], 128);
     while (zc > 4 && cols * ((a.nq[2] + zc - 1) / zc) * threads < (zc > 8 ? 1LL << 18 : 1LL << 16))
       zc = (zc + 1) / 2;

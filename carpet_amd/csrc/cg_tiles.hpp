@@ -10,7 +10,9 @@
 //   1. the coarse plane window (tile + stencil halo, clipped to the region's
 //      exact source footprint) is loaded into LDS with coalesced x-rows;
 //   2. x-pass: every coarse row of the window is interpolated to both fine
-//      x children of each base (LDS -> LDS);
+//      x children of each base (LDS -> LDS; kinds whose children come in
+//      pairs, ENO, evaluate the two children between two cells together, here
+//      and in the other passes);
 //   3. y-pass: every fine x column is interpolated to both fine y children
 //      of each base; the results stay in registers in a ring of the last R
 //      coarse planes;
@@ -188,7 +190,10 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
   const int f0 = a.off[0] - a.sx + tx * FX;
   const int qx0 = f0 >> 1;
   const bool odd = f0 & 1;
-  const int qy0 = a.qlo[1] + ty * CY;
+  // tile row j is fine point fy0 + j: fy0 even, or odd for kinds whose
+  // children come in pairs, so that a thread's two rows are a pair
+  const int ry0 = ty * 2 * CY - a.sy;
+  const int qy0 = (a.off[1] + ry0) >> 1;
   const int qz0 = a.qlo[2] + tz * a.zchunk;
   const int qz1 = min(qz0 + a.zchunk, a.qlo[2] + a.nq[2]) - 1;
 
@@ -237,6 +242,10 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
 #pragma unroll
       for (int m = 0; m < IPT; ++m)
         ring[tl][i][m][0] = ring[tl][i][m][1] = CT(0);
+  // paired kinds keep the z differences of the last ND planes where the
+  // registers allow it (one time level)
+  constexpr int DZ = L::PAIRED && NTL == 1 ? NTL : 0;
+  double dz[DZ > 0 ? DZ : 1][L::PAIRED ? R : 1][IPT][2];
 
   auto prologue = [&](auto Sc) -> bool {
     constexpr int S = decltype(Sc)::value;
@@ -289,17 +298,41 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
         v[2 * m] = p.x;
         v[2 * m + 1] = p.y;
       }
-      constexpr int O0 = L::TMIN[0] - L::TMINALL, O1 = L::TMIN[1] - L::TMINALL;
-      const CT b = line_apply<L, 1, CT>([&](int t) { return v[O1 + t]; });
-      const CT c = line_apply<L, 0, CT>([&](int t) { return v[1 + O0 + t]; });
-      const CT d = line_apply<L, 1, CT>([&](int t) { return v[1 + O1 + t]; });
       C2 lo, hi;
-      if (odd) {
-        lo.x = b, lo.y = c, hi.x = d;
-        hi.y = line_apply<L, 0, CT>([&](int t) { return v[2 + O0 + t]; });
+      if constexpr (L::PAIRED) {
+        // interval k lies right of base q0 - 1 + k, its values from v[k] on
+        double d[L::ND + 2], lf[3], rt[3];
+#pragma unroll
+        for (int k = 0; k < L::ND + 2; ++k)
+          d[k] = L::diff([&](int t) { return v[k + t]; });
+        auto interval = [&](auto kc) {
+          constexpr int k = decltype(kc)::value;
+          double dk[L::ND];
+#pragma unroll
+          for (int t = 0; t < L::ND; ++t)
+            dk[t] = d[k + t];
+          L::pair([&](int t) { return v[k + t]; }, dk, rt[k], lf[k]);
+        };
+        interval(std::integral_constant<int, 1>{});
+        interval(std::integral_constant<int, 2>{});
+        if (odd) {
+          lo.x = rt[1], lo.y = lf[1], hi.x = rt[2], hi.y = lf[2];
+        } else {
+          interval(std::integral_constant<int, 0>{});
+          lo.x = lf[0], lo.y = rt[1], hi.x = lf[1], hi.y = rt[2];
+        }
       } else {
-        lo.x = line_apply<L, 0, CT>([&](int t) { return v[O0 + t]; });
-        lo.y = b, hi.x = c, hi.y = d;
+        constexpr int O0 = L::TMIN[0] - L::TMINALL, O1 = L::TMIN[1] - L::TMINALL;
+        const CT b = line_apply<L, 1, CT>([&](int t) { return v[O1 + t]; });
+        const CT c = line_apply<L, 0, CT>([&](int t) { return v[1 + O0 + t]; });
+        const CT d = line_apply<L, 1, CT>([&](int t) { return v[1 + O1 + t]; });
+        if (odd) {
+          lo.x = b, lo.y = c, hi.x = d;
+          hi.y = line_apply<L, 0, CT>([&](int t) { return v[2 + O0 + t]; });
+        } else {
+          lo.x = line_apply<L, 0, CT>([&](int t) { return v[O0 + t]; });
+          lo.y = b, hi.x = c, hi.y = d;
+        }
       }
       *reinterpret_cast<C2 *>(&X[tl][r][2 * q0]) = lo;
       *reinterpret_cast<C2 *>(&X[tl][r][2 * q0 + 2]) = hi;
@@ -317,39 +350,99 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
 #pragma unroll
       for (int tl = 0; tl < NTL; ++tl) {
         const CT *col = &X[tl][qy - L::TMINALL][fx];
-        ring[tl][J][m][0] = line_apply<L, 0, CT>([&](int t) { return col[(L::TMIN[0] + t) * FX]; });
-        ring[tl][J][m][1] = line_apply<L, 1, CT>([&](int t) { return col[(L::TMIN[1] + t) * FX]; });
-      }
-    }
-    auto emit = [&](auto PZc) {
-      constexpr int PZ = decltype(PZc)::value;
-      constexpr int NTP = L::NTAP[PZ];
-      constexpr int TMAX = L::TMIN[PZ] + NTP - 1;
-      const int base = p - TMAX;
-      if (base < qz0 || base > qz1)
-        return;
-      const int fz = 2 * base + PZ - a.off[2];
-      if (fz < 0 || fz >= a.n[2])
-        return;
+        if constexpr (L::PAIRED) {
+          double v[R], d[L::ND];
 #pragma unroll
-      for (int m = 0; m < IPT; ++m) {
+          for (int t = 0; t < R; ++t)
+            v[t] = col[(L::TMIN[1] + t) * FX];
 #pragma unroll
-        for (int py = 0; py < 2; ++py) {
-          const int fy = 2 * (qy0 + qyl + NQY * m) + py - a.off[1];
-          double v[NTL];
-#pragma unroll
-          for (int tl = 0; tl < NTL; ++tl)
-            v[tl] = (double)line_apply<L, PZ, CT>(
-                [&](int t) { return ring[tl][(J - NTP + 1 + t + 2 * R) % R][m][py]; });
-          // time interpolation in FP64 in every precision mode
-          const double out = time_combine<NTL>(v, a.s, a.s2, a.l0, a.teno, a.nlev);
-          if (xin && fy >= 0 && fy < a.n[1])
-            __builtin_nontemporal_store((TS)out, &((CG_GLOBAL TS *)a.dst)[gfx + a.dj * fy + a.dk * fz]);
+          for (int k = 0; k < L::ND; ++k)
+            d[k] = L::diff([&](int t) { return v[k + t]; });
+          L::pair([&](int t) { return v[t]; }, d, ring[tl][J][m][0], ring[tl][J][m][1]);
+        } else {
+          ring[tl][J][m][0] = line_apply<L, 0, CT>([&](int t) { return col[(L::TMIN[0] + t) * FX]; });
+          ring[tl][J][m][1] = line_apply<L, 1, CT>([&](int t) { return col[(L::TMIN[1] + t) * FX]; });
         }
       }
+    }
+    // fine z plane of parity PZ whose last coarse plane is p, -1 if it is not
+    // this chunk's
+    auto fine_z = [&](auto PZc) -> int {
+      constexpr int PZ = decltype(PZc)::value;
+      const int base = p - (L::TMIN[PZ] + L::NTAP[PZ] - 1);
+      const int fz = 2 * base + PZ - a.off[2];
+      return base >= qz0 && base <= qz1 && fz >= 0 && fz < a.n[2] ? fz : -1;
     };
-    emit(std::integral_constant<int, 0>{});
-    emit(std::integral_constant<int, 1>{});
+    // v: the values of the time levels at a point of row py of base row m
+    auto put = [&](int fz, int m, int py, const double *v) {
+      const int fy = ry0 + 2 * (qyl + NQY * m) + py;
+      // time interpolation in FP64 in every precision mode
+      const double out = time_combine<NTL>(v, a.s, a.s2, a.l0, L::ENO_TIME ? a.teno : 0, a.nlev);
+      if (xin && fy >= 0 && fy < a.n[1])
+        __builtin_nontemporal_store((TS)out, &((CG_GLOBAL TS *)a.dst)[gfx + a.dj * fy + a.dk * fz]);
+    };
+    if constexpr (L::PAIRED) {
+      // difference that ends with this plane: each serves ND intervals
+      if constexpr (DZ > 0)
+#pragma unroll
+        for (int m = 0; m < IPT; ++m)
+#pragma unroll
+          for (int py = 0; py < 2; ++py)
+#pragma unroll
+            for (int tl = 0; tl < NTL; ++tl)
+              dz[tl][J % L::ND][m][py] =
+                  L::diff([&](int t) { return ring[tl][(J - L::ND + t + 2 * R) % R][m][py]; });
+      const int z1 = fine_z(std::integral_constant<int, 1>{}), z0 = fine_z(std::integral_constant<int, 0>{});
+      if (z0 < 0 && z1 < 0)
+        return;
+#pragma unroll
+      for (int m = 0; m < IPT; ++m)
+#pragma unroll
+        for (int py = 0; py < 2; ++py) {
+          double hi[NTL], lo[NTL];
+#pragma unroll
+          for (int tl = 0; tl < NTL; ++tl) {
+            auto v = [&](int t) { return ring[tl][(J + 1 + t) % R][m][py]; };
+            double d[L::ND];
+#pragma unroll
+            for (int k = 0; k < L::ND; ++k)
+              d[k] = DZ > 0 ? dz[tl][DZ > 0 ? (J + 1 + k) % L::ND : 0][m][py]
+                            : L::diff([&](int t) { return v(k + t); });
+            L::pair(v, d, hi[tl], lo[tl]);
+          }
+          if (z1 >= 0)
+            put(z1, m, py, hi);
+          if (z0 >= 0)
+            put(z0, m, py, lo);
+        }
+      return;
+    } else {
+      auto emit = [&](auto PZc) {
+        constexpr int PZ = decltype(PZc)::value;
+        constexpr int NTP = L::NTAP[PZ];
+        constexpr int TMAX = L::TMIN[PZ] + NTP - 1;
+        const int base = p - TMAX;
+        if (base < qz0 || base > qz1)
+          return;
+        const int fz = 2 * base + PZ - a.off[2];
+        if (fz < 0 || fz >= a.n[2])
+          return;
+  #pragma unroll
+        for (int m = 0; m < IPT; ++m) {
+  #pragma unroll
+          for (int py = 0; py < 2; ++py) {
+            double v[NTL];
+  #pragma unroll
+            for (int tl = 0; tl < NTL; ++tl)
+              v[tl] = (double)line_apply<L, PZ, CT>(
+                  [&](int t) { return ring[tl][(J - NTP + 1 + t + 2 * R) % R][m][py]; });
+            put(fz, m, py, v);
+          }
+        }
+      };
+      emit(std::integral_constant<int, 0>{});
+      emit(std::integral_constant<int, 1>{});
+    }
   };
 
   int c = c0;
@@ -862,9 +955,11 @@ template <int NTL> struct TileShape<NTL, 3, 0> {
   static constexpr int CX = 4, CY = 16, IPT = 1;
 };
 // the pipelined schedule (double-buffered window and x-pass results) where
-// its LDS fits the 64 KB of a static allocation, else two barriers per plane
+// its LDS fits 64 KB, for kinds with paired children 80 KB (two workgroups a
+// CU: 8 x 320^3 cell ENO<3> with 3 levels, 69 KB, 2.67 ms pipelined, 2.74 with
+// two barriers a plane), else two barriers per plane
 template <class L, int NTL, int CX, int CY> constexpr int pipe_fits() {
-  return TensorLds<L, NTL, CX, CY, 2>::TOTAL * 8 <= 65536 ? 1 : 0;
+  return TensorLds<L, NTL, CX, CY, 2>::TOTAL * 8 <= (L::PAIRED ? 81920 : 65536) ? 1 : 0;
 }
 template <class L, int NTL, int CX, int CY> constexpr int tile_lds() {
   return TensorLds<L, NTL, CX, CY, pipe_fits<L, NTL, CX, CY>() ? 2 : 1>::TOTAL;

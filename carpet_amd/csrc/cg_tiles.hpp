@@ -153,8 +153,17 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
   using WT = std::conditional_t<TF, CT, TS>; // LDS window type
   constexpr int FX = 2 * CX;
   constexpr int NT = FX * CY / IPT;
-  constexpr int NQY = NT / FX;
-  static_assert(NQY * IPT == CY, "tile rows must divide among threads");
+  // what a thread with IPT = 2 owns: two neighbouring fine columns of one base
+  // row where the arrays are FP32, so that the y-pass reads LDS and the
+  // emission writes memory in pairs (8 x 384^3, 3 levels: 633 against 595 us
+  // a pass; 8 x 198x178x158: 71.7 and 72.7; odd widths write a row's last
+  // line in two parts: 197 wide 72.5 and 77.7), else two base rows of one
+  // column (in FP64 pairs are 16-byte stores: 8 x 231x165x297 order 3, 179 us
+  // with rows, 195 with columns)
+  constexpr bool COLS = IPT == 2 && sizeof(TS) == 4;
+  constexpr int NC = COLS ? 2 : 1;     // columns of a thread
+  constexpr int NQY = NT / (FX / NC);  // base rows of the threads' first items
+  static_assert(IPT <= 2 && NQY * (IPT / NC) == CY, "tile rows must divide among threads");
   static_assert(CX % 2 == 0, "the x-pass takes two bases per thread");
   constexpr int NB = PIPE ? 2 : 1;
   using LD = TensorLds<L, NTL, CX, CY, NB>;
@@ -204,9 +213,16 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
   const int c1 = min(qz1 + L::TMAXALL, a.fhi[2]);
 
   const int tid = threadIdx.x;
-  const int fx = tid % FX, qyl = tid / FX;
+  const int fx = tid % (FX / NC) * NC, qyl = tid / (FX / NC);
   const int gfx = tx * FX + fx - a.sx;
   const bool xin = gfx >= 0 && gfx < a.n[0];
+  // COLS: pairs of columns are aligned in every row; the region begins or
+  // ends inside a pair
+  const int px0 = tx * FX - a.sx; // the tile's first column
+  const bool pairs = COLS && (((uintptr_t)a.dst + px0 * (long long)sizeof(TS)) & (2 * sizeof(TS) - 1)) == 0 &&
+                     ((a.dj | a.dk) & 1) == 0;
+  const bool edge = (px0 < 0 && (px0 & 1)) || (px0 + FX > a.n[0] && ((a.n[0] - px0) & 1));
+  const bool xin1 = COLS && gfx + 1 >= 0 && gfx + 1 < a.n[0];
 
   // this thread's share of the plane window: offsets into the source plane
   // (or -1 outside the clipped footprint)
@@ -344,26 +360,43 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
   auto ypass_emit = [&](auto Bc, auto Jc, int p) {
     constexpr int J = decltype(Jc)::value;
     auto X = Xbuf(decltype(Bc)::value);
+    // both children of a base row from its coarse rows: at(t) is the value at
+    // row offset t
+    auto children = [&](auto at, CT &c0, CT &c1) {
+      if constexpr (L::PAIRED) {
+        double v[R], d[L::ND];
 #pragma unroll
-    for (int m = 0; m < IPT; ++m) {
-      const int qy = qyl + NQY * m;
+        for (int t = 0; t < R; ++t)
+          v[t] = at(L::TMIN[1] + t);
+#pragma unroll
+        for (int k = 0; k < L::ND; ++k)
+          d[k] = L::diff([&](int t) { return v[k + t]; });
+        L::pair([&](int t) { return v[t]; }, d, c0, c1);
+      } else {
+        c0 = line_apply<L, 0, CT>([&](int t) { return at(L::TMIN[0] + t); });
+        c1 = line_apply<L, 1, CT>([&](int t) { return at(L::TMIN[1] + t); });
+      }
+    };
+    if constexpr (COLS) {
 #pragma unroll
       for (int tl = 0; tl < NTL; ++tl) {
-        const CT *col = &X[tl][qy - L::TMINALL][fx];
-        if constexpr (L::PAIRED) {
-          double v[R], d[L::ND];
+        const CT *col = &X[tl][qyl - L::TMINALL][fx];
+        constexpr int NV = L::TMAXALL - L::TMINALL + 1;
+        typename Pair<CT>::T w[NV];
 #pragma unroll
-          for (int t = 0; t < R; ++t)
-            v[t] = col[(L::TMIN[1] + t) * FX];
-#pragma unroll
-          for (int k = 0; k < L::ND; ++k)
-            d[k] = L::diff([&](int t) { return v[k + t]; });
-          L::pair([&](int t) { return v[t]; }, d, ring[tl][J][m][0], ring[tl][J][m][1]);
-        } else {
-          ring[tl][J][m][0] = line_apply<L, 0, CT>([&](int t) { return col[(L::TMIN[0] + t) * FX]; });
-          ring[tl][J][m][1] = line_apply<L, 1, CT>([&](int t) { return col[(L::TMIN[1] + t) * FX]; });
-        }
+        for (int t = 0; t < NV; ++t)
+          w[t] = *reinterpret_cast<const typename Pair<CT>::T *>(col + (L::TMINALL + t) * FX);
+        children([&](int t) { return w[t - L::TMINALL].x; }, ring[tl][J][0][0], ring[tl][J][0][1]);
+        children([&](int t) { return w[t - L::TMINALL].y; }, ring[tl][J][IPT - 1][0], ring[tl][J][IPT - 1][1]);
       }
+    } else {
+#pragma unroll
+      for (int m = 0; m < IPT; ++m)
+#pragma unroll
+        for (int tl = 0; tl < NTL; ++tl) {
+          const CT *col = &X[tl][qyl + NQY * m - L::TMINALL][fx];
+          children([&](int t) { return col[t * FX]; }, ring[tl][J][m][0], ring[tl][J][m][1]);
+        }
     }
     // fine z plane of parity PZ whose last coarse plane is p, -1 if it is not
     // this chunk's
@@ -373,13 +406,34 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
       const int fz = 2 * base + PZ - a.off[2];
       return base >= qz0 && base <= qz1 && fz >= 0 && fz < a.n[2] ? fz : -1;
     };
-    // v: the values of the time levels at a point of row py of base row m
-    auto put = [&](int fz, int m, int py, const double *v) {
-      const int fy = ry0 + 2 * (qyl + NQY * m) + py;
-      // time interpolation in FP64 in every precision mode
-      const double out = time_combine<NTL>(v, a.s, a.s2, a.l0, L::ENO_TIME ? a.teno : 0, a.nlev);
-      if (xin && fy >= 0 && fy < a.n[1])
-        __builtin_nontemporal_store((TS)out, &((CG_GLOBAL TS *)a.dst)[gfx + a.dj * fy + a.dk * fz]);
+    // time interpolation in FP64 in every precision mode
+    auto combine = [&](const double *v) {
+      return time_combine<NTL>(v, a.s, a.s2, a.l0, L::ENO_TIME ? a.teno : 0, a.nlev);
+    };
+    // this thread's points of plane fz: fine row py of its base row(s)
+    auto put = [&](int fz, int py, const double *out) {
+#pragma unroll
+      for (int m = 0; m < IPT / NC; ++m) {
+        const int fy = ry0 + 2 * (qyl + NQY * m) + py;
+        const bool yin = fy >= 0 && fy < a.n[1];
+        const auto d = (CG_GLOBAL TS *)a.dst + (gfx + a.dj * fy + a.dk * fz);
+        if constexpr (COLS) {
+          typedef TS pair_t __attribute__((ext_vector_type(2)));
+          if (pairs) {
+            if (yin && xin && xin1)
+              __builtin_nontemporal_store(pair_t{(TS)out[0], (TS)out[IPT - 1]}, (CG_GLOBAL pair_t *)d);
+            if (!edge)
+              continue;
+          }
+          if (yin && xin1 && !(pairs && xin))
+            __builtin_nontemporal_store((TS)out[IPT - 1], d + 1);
+          if (yin && xin && !(pairs && xin1))
+            __builtin_nontemporal_store((TS)out[0], d);
+          continue;
+        }
+        if (yin && xin)
+          __builtin_nontemporal_store((TS)out[m], d);
+      }
     };
     if constexpr (L::PAIRED) {
       // difference that ends with this plane: each serves ND intervals
@@ -396,9 +450,10 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
       if (z0 < 0 && z1 < 0)
         return;
 #pragma unroll
-      for (int m = 0; m < IPT; ++m)
+      for (int py = 0; py < 2; ++py) {
+        double o1[IPT], o0[IPT];
 #pragma unroll
-        for (int py = 0; py < 2; ++py) {
+        for (int m = 0; m < IPT; ++m) {
           double hi[NTL], lo[NTL];
 #pragma unroll
           for (int tl = 0; tl < NTL; ++tl) {
@@ -410,11 +465,14 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
                             : L::diff([&](int t) { return v(k + t); });
             L::pair(v, d, hi[tl], lo[tl]);
           }
-          if (z1 >= 0)
-            put(z1, m, py, hi);
-          if (z0 >= 0)
-            put(z0, m, py, lo);
+          o1[m] = combine(hi);
+          o0[m] = combine(lo);
         }
+        if (z1 >= 0)
+          put(z1, py, o1);
+        if (z0 >= 0)
+          put(z0, py, o0);
+      }
       return;
     } else {
       auto emit = [&](auto PZc) {
@@ -427,17 +485,19 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
         const int fz = 2 * base + PZ - a.off[2];
         if (fz < 0 || fz >= a.n[2])
           return;
-  #pragma unroll
-        for (int m = 0; m < IPT; ++m) {
-  #pragma unroll
-          for (int py = 0; py < 2; ++py) {
+#pragma unroll
+        for (int py = 0; py < 2; ++py) {
+          double out[IPT];
+#pragma unroll
+          for (int m = 0; m < IPT; ++m) {
             double v[NTL];
-  #pragma unroll
+#pragma unroll
             for (int tl = 0; tl < NTL; ++tl)
               v[tl] = (double)line_apply<L, PZ, CT>(
                   [&](int t) { return ring[tl][(J - NTP + 1 + t + 2 * R) % R][m][py]; });
-            put(fz, m, py, v);
+            out[m] = combine(v);
           }
+          put(fz, py, out);
         }
       };
       emit(std::integral_constant<int, 0>{});

@@ -295,6 +295,51 @@ int small_tiles(const ProlongPlan &p, int ntl, int prec) {
   return (sh == 3 ? b3 : b2) * 1.3 <= big ? sh : 0;
 }
 
+// Regions of one kernel whose shapes fall into three classes or more run as
+// one class on the 8x8 tiles where the chip holds few rounds of those: every
+// class beyond the first costs a launch, a fork and a join of streams, and a
+// tail.  Up to 32 tiles a CU that is more than the better shapes give; up to
+// 128 only if the small tiles keep at most a quarter more lanes busy.  (In
+// several classes against one: 300 regions of 5-31 points per axis x 3, order
+// 3, 2 levels 62 against 29 us, from a graph 45 against 33; a 3-level
+// hierarchy of 64^3 coarse points x 4 116 against 86 us, of 128^3 x 12, which
+// keeps its classes, 475 against 488 us; 432 boxes x 4 1.274 against 1.240
+// ms; 1000 regions of 8-60 points 626 against 598 us.)
+constexpr long long MERGE_POINTS = 1 << 18; // per region
+void merge_small_classes(const std::vector<Transfer> &tr, std::vector<Group> &per, int ncu) {
+  std::vector<char> done(per.size(), 0);
+  for (size_t i = 0; i < per.size(); ++i) {
+    if (done[i] || !per[i].is_tensor || per[i].prec != CG_PREC_F64)
+      continue;
+    std::vector<size_t> same;
+    long long items = 0;
+    double busy = 0, busy8 = 0;
+    bool small = true;
+    int seen = 0; // shapes, a bit each
+    for (size_t j = i; j < per.size(); ++j) {
+      const Group &g = per[j];
+      if (!g.is_tensor || g.phase != per[i].phase || g.kind != per[i].kind || g.order != per[i].order ||
+          g.ntl != per[i].ntl || g.prec != per[i].prec)
+        continue;
+      same.push_back(j);
+      done[j] = 1;
+      seen |= 1 << (g.small ? g.small : g.bigsh);
+      const TensorArgs &a = tr[j].pr.t;
+      small = small && tr[j].dst_points() <= MERGE_POINTS;
+      const int span = line_span(g.kind, g.order);
+      busy += tile_busy(a, g.ntl, g.prec, span, g.small ? g.small : g.bigsh);
+      busy8 += tile_busy(a, g.ntl, g.prec, span, 2);
+      items += (long long)tiles_x(a, 8, tile_shift(a, 8, 8)) * tiles_y(a, 8) * ((a.nq[2] + 7) / 8);
+    }
+    if (small && __builtin_popcount((unsigned)seen) >= 3 &&
+        items <= (busy8 <= 1.25 * busy ? 128LL : 32LL) * ncu)
+      for (size_t j : same) {
+        per[j].small = 2;
+        per[j].bigsh = 0;
+      }
+  }
+}
+
 // one transfer's descriptor in launch l: a tensor transfer resolved to one
 // time level (its target time matches level 0 exactly) inside a class of
 // more levels keeps nlev = 1 and reads level 0 for every level slot; a
@@ -481,7 +526,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
                        int only) {
   batch_device_free(dev);
   // group transfers by (phase, kernel)
-  std::vector<Group> groups;
+  std::vector<Group> groups, per;
   for (size_t i = 0; i < tr.size(); ++i) {
     Group g{};
     g.phase = phase[i];
@@ -518,6 +563,18 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
              : tr[i].pr.kind == PK_STAGGER ? PO_STAGGER
                                            : PO_TVD;
     }
+    per.push_back(g);
+  }
+  int dev_id = 0, ncu = 0;
+  hipError_t he = hipGetDevice(&dev_id);
+  if (he != hipSuccess)
+    return hip_error(he, "hipGetDevice");
+  he = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev_id);
+  if (he != hipSuccess)
+    return hip_error(he, "hipDeviceGetAttribute");
+  merge_small_classes(tr, per, ncu);
+  for (size_t i = 0; i < tr.size(); ++i) {
+    const Group &g = per[i];
     auto it = std::find_if(groups.begin(), groups.end(), [&](const Group &x) { return x.same(g); });
     if (it == groups.end()) {
       groups.push_back(g);
@@ -527,14 +584,6 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
   }
   std::stable_sort(groups.begin(), groups.end(),
                    [](const Group &a, const Group &b) { return a.phase < b.phase; });
-
-  int dev_id = 0, ncu = 0;
-  hipError_t he = hipGetDevice(&dev_id);
-  if (he != hipSuccess)
-    return hip_error(he, "hipGetDevice");
-  he = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev_id);
-  if (he != hipSuccess)
-    return hip_error(he, "hipDeviceGetAttribute");
 
   // host image of the blob: per launch, descriptors then items (8-byte aligned)
   std::vector<char> host;

@@ -304,7 +304,9 @@ int small_tiles(const ProlongPlan &p, int ntl, int prec) {
 // 3, 2 levels 62 against 29 us, from a graph 45 against 33; a 3-level
 // hierarchy of 64^3 coarse points x 4 116 against 86 us, of 128^3 x 12, which
 // keeps its classes, 475 against 488 us; 432 boxes x 4 1.274 against 1.240
-// ms; 1000 regions of 8-60 points 626 against 598 us.)
+// ms; 1000 regions of 8-60 points 626 against 598 us.)  Fewer than 128 regions
+// keep their classes, which a caller can run beside each other or in turn
+// (cg_batch_set_phase_mode).
 constexpr long long MERGE_POINTS = 1 << 18; // per region
 void merge_small_classes(const std::vector<Transfer> &tr, std::vector<Group> &per, int ncu) {
   std::vector<char> done(per.size(), 0);
@@ -331,7 +333,7 @@ void merge_small_classes(const std::vector<Transfer> &tr, std::vector<Group> &pe
       busy8 += tile_busy(a, g.ntl, g.prec, span, 2);
       items += (long long)tiles_x(a, 8, tile_shift(a, 8, 8)) * tiles_y(a, 8) * ((a.nq[2] + 7) / 8);
     }
-    if (small && __builtin_popcount((unsigned)seen) >= 3 &&
+    if (small && __builtin_popcount((unsigned)seen) >= 3 && same.size() >= 128 &&
         items <= (busy8 <= 1.25 * busy ? 128LL : 32LL) * ncu)
       for (size_t j : same) {
         per[j].small = 2;

@@ -25,10 +25,11 @@ def test_one_class_matches_oracle(cent, op, order, ntl, large):
         w.arrays[f"c{tl}"] = ArraySpec(cbox, seed=700 + tl)
     # thin in x, thin in x and y, a cube, one column wide, wide and flat
     ext = [(3, 50, 44), (6, 6, 40), (30, 30, 30), (1, 1, 1), (70, 20, 24), (64, 9, 31), (2, 60, 2)]
+    ext = ext * 19  # 133 regions
     if large:
         ext.append((90, 80, 64))
     for r, n in enumerate(ext):
-        lo = (5 + r, 4 + 2 * r, 3 + r % 2)
+        lo = (5 + r % 19, 4 + r % 17, 3 + r % 2)
         reg = Box(tuple(fo + fs * l for l in lo), tuple(fo + fs * (l + k - 1) for l, k in zip(lo, n)), (fs,) * 3)
         w.arrays[f"f{r}"] = ArraySpec(reg.expand((3, 3, 3), (3, 3, 3)), owned=reg, seed=750 + r)
         w.steps.append(Transfer(f"f{r}", f"f{r}", [f"c{tl}" for tl in range(ntl)], [0.0, -1.0, -2.0][:ntl], reg, reg,

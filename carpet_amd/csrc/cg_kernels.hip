@@ -59,7 +59,10 @@ int launch_tensor(int kind, int order, int ntl, int prec, const TensorArgs &a,
 void point_rows(PointArgs &a) {
   const int s = (int)(reinterpret_cast<uintptr_t>(a.dst) / 8 % 16);
   const long long w = ((long long)s + a.n[0] + 15) / 16 * 16;
-  const bool lines = a.dj % 16 == 0 && a.dk % 16 == 0 && w <= 2LL * a.n[0];
+  // (regions of 2^30 slots and more stay flat: no fewer fit the 31-bit slot
+  // numbers than points did)
+  const bool lines =
+      a.dj % 16 == 0 && a.dk % 16 == 0 && w <= 2LL * a.n[0] && w * a.n[1] < (1LL << 30) / std::max(1, a.n[2]);
   a.sx = lines ? s : 0;
   a.nxp = lines ? (int)w : a.n[0];
   a.fx = make_fastdiv((unsigned)a.nxp);

@@ -382,8 +382,12 @@ PointArgs point_desc(const BatchLaunch &l, const Transfer &t, int sx = 0, int nx
   }
   long long u[3];
   point_units(l, a, u);
-  a.fx = make_fastdiv((unsigned)u[0]);
-  a.fxy = make_fastdiv((unsigned)(u[0] * u[1]));
+  // (planes of 2^31 units and more are refused: no divisor, which cut to 32
+  // bits may be 0)
+  if (u[0] * u[1] < (1LL << 31)) {
+    a.fx = make_fastdiv((unsigned)u[0]);
+    a.fxy = make_fastdiv((unsigned)(u[0] * u[1]));
+  }
   return a;
 }
 

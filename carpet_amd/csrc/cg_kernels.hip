@@ -65,8 +65,6 @@ void point_rows(PointArgs &a) {
       a.dj % 16 == 0 && a.dk % 16 == 0 && w <= 2LL * a.n[0] && w * a.n[1] < (1LL << 30) / std::max(1, a.n[2]);
   a.sx = lines ? s : 0;
   a.nxp = lines ? (int)w : a.n[0];
-  a.fx = make_fastdiv((unsigned)a.nxp);
-  a.fxy = make_fastdiv((unsigned)((long long)a.nxp * a.n[1]));
 }
 
 template <int OP>
@@ -122,6 +120,8 @@ int launch_point(int op, const PointArgs &a0, hipStream_t s) {
   const long long nxy = (long long)a.nxp * a.n[1];
   if (nxy <= 0 || a.n[2] <= 0 || nxy >= (1LL << 32) / 2)
     return -1;
+  a.fx = make_fastdiv((unsigned)a.nxp);
+  a.fxy = make_fastdiv((unsigned)nxy);
   const unsigned gx = (unsigned)((nxy + 255) / 256);
   const unsigned gy = (unsigned)(a.n[2] < 65535 ? a.n[2] : 65535);
   dim3 grid(gx, gy), block(256);

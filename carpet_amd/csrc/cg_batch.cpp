@@ -43,6 +43,7 @@ struct cg_batch {
   std::vector<int> phase;
   std::vector<int> prec;
   std::vector<int> cls_ntl; // time levels of each transfer's launch class
+  std::vector<char> shapes; // tile shape of each transfer's launch class (set by finalize)
   std::vector<BatchAddArgs> args;
   cg::BatchDevice dev;
   cg::TuneMap tuned;
@@ -190,7 +191,8 @@ int cg_batch_finalize(cg_batch *b, int tile_cfg) {
   if (b->finalized)
     return set_error(CG_ERR_STATE, "batch already finalized");
   b->tile_cfg = tile_cfg;
-  int e = batch_device_build(b->dev, b->transfers, b->phase, b->prec, b->cls_ntl, tile_cfg, &b->tuned);
+  b->shapes.clear();
+  int e = batch_device_build(b->dev, b->transfers, b->phase, b->prec, b->cls_ntl, b->shapes, tile_cfg, &b->tuned);
   if (e)
     return e;
   index_launches(b);
@@ -331,8 +333,8 @@ extern "C" int cg_batch_autotune(cg_batch *b, cg_stream_t stream, int reps,
       TuneMap trial = b->tuned;
       trial[l.key] = c;
       BatchDevice one;
-      int e = batch_device_build(one, b->transfers, b->phase, b->prec, b->cls_ntl, b->tile_cfg, &trial,
-                                 (int)i);
+      int e = batch_device_build(one, b->transfers, b->phase, b->prec, b->cls_ntl, b->shapes, b->tile_cfg,
+                                 &trial, (int)i);
       float ms = 0;
       if (!e && one.launches.size() != 1)
         e = set_error(CG_ERR_STATE, "tuner: launch %zu did not build alone", i);
@@ -376,7 +378,7 @@ extern "C" int cg_batch_autotune(cg_batch *b, cg_stream_t stream, int reps,
     }
     b->tuned[l.key] = bestc;
   }
-  int e = batch_device_build(b->dev, b->transfers, b->phase, b->prec, b->cls_ntl, b->tile_cfg, &b->tuned);
+  int e = batch_device_build(b->dev, b->transfers, b->phase, b->prec, b->cls_ntl, b->shapes, b->tile_cfg, &b->tuned);
   if (e)
     return e;
   index_launches(b);

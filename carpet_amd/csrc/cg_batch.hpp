@@ -85,11 +85,14 @@ struct BatchDevice {
 // tile_cfg selects the z chunk of tensor tiles in coarse bases (0 = whole
 // region, < 0 = automatic); cls_ntl: per transfer the time levels of its
 // launch class (a tensor transfer resolved to fewer levels -- an exact time
-// match -- runs in its class with nlev = 1); only >= 0 builds launch `only`
-// of the full build alone (the tuner's trials)
+// match -- runs in its class with nlev = 1); shapes: per transfer the tile
+// shape of its launch class, chosen by the first build (an empty vector) and
+// kept by the later ones, so that the tuner's trials and rebuilds have the
+// same classes also after new storage has moved a region to another alignment;
+// only >= 0 builds launch `only` of the full build alone (the tuner's trials)
 int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
                        const std::vector<int> &phase, const std::vector<int> &prec,
-                       const std::vector<int> &cls_ntl, int tile_cfg,
+                       const std::vector<int> &cls_ntl, std::vector<char> &shapes, int tile_cfg,
                        const TuneMap *tuned = nullptr, int only = -1);
 // the descriptor array of launch l from the current transfers, in the
 // layout batch_device_build uploads (the per-step parameter path rewrites

@@ -528,10 +528,11 @@ void batch_launch_descs(const BatchLaunch &l, const std::vector<Transfer> &tr, c
 
 int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
                        const std::vector<int> &phase, const std::vector<int> &prec,
-                       const std::vector<int> &cls_ntl, int tile_cfg, const TuneMap *tuned,
-                       int only) {
+                       const std::vector<int> &cls_ntl, std::vector<char> &shapes, int tile_cfg,
+                       const TuneMap *tuned, int only) {
   batch_device_free(dev);
   // group transfers by (phase, kernel)
+  const bool chosen = !shapes.empty();
   std::vector<Group> groups, per;
   for (size_t i = 0; i < tr.size(); ++i) {
     Group g{};
@@ -540,7 +541,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     if (tr[i].is_prolong && tr[i].pr.kind != PK_TVD && tr[i].pr.kind != PK_MONO5 &&
         tr[i].pr.kind != PK_STAGGER) {
       g.is_tensor = 1;
-      g.small = small_tiles(tr[i].pr, cls_ntl[i], prec[i]);
+      g.small = chosen ? 0 : small_tiles(tr[i].pr, cls_ntl[i], prec[i]);
       // the large shape that keeps fewer lanes busy on this region -- tiles x
       // (planes + stencil span) x (tile width) x (tile rows + span), the work
       // of the window loads and of the x- and y-passes -- with a 25% margin
@@ -550,7 +551,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
       // regions of 8-96 points per axis, 1.8% and 1.2% on the level steps
       // of the 3-level and the 2000-box hierarchies.
       g.bigsh = 0;
-      if (!g.small) {
+      if (!chosen && !g.small) {
         const int span = line_span(tr[i].pr.kind, tr[i].pr.order);
         const double b0 = tile_busy(tr[i].pr.t, cls_ntl[i], prec[i], span, 0);
         const double b1 = tile_busy(tr[i].pr.t, cls_ntl[i], prec[i], span, 1);
@@ -578,8 +579,17 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
   he = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev_id);
   if (he != hipSuccess)
     return hip_error(he, "hipDeviceGetAttribute");
-  merge_small_classes(tr, per, ncu);
+  if (!chosen) {
+    merge_small_classes(tr, per, ncu);
+    shapes.resize(tr.size());
+  }
   for (size_t i = 0; i < tr.size(); ++i) {
+    if (chosen) {
+      per[i].small = shapes[i] >= 2 ? shapes[i] : 0;
+      per[i].bigsh = shapes[i] == 1;
+    } else {
+      shapes[i] = (char)(per[i].small ? per[i].small : per[i].bigsh);
+    }
     const Group &g = per[i];
     auto it = std::find_if(groups.begin(), groups.end(), [&](const Group &x) { return x.same(g); });
     if (it == groups.end()) {

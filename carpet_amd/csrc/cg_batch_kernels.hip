@@ -375,7 +375,10 @@ PointArgs point_desc(const BatchLaunch &l, const Transfer &t, int sx = 0, int nx
     a.ntl = 1;
     a.s[0] = 1.0;
   }
-  point_rows(a);
+  a.sx = 0;
+  a.nxp = a.n[0];
+  if (l.op != PO_TVD)
+    point_rows(l.op, a);
   if (nxp > 0) {
     a.sx = sx;
     a.nxp = nxp;

@@ -51,18 +51,36 @@ int launch_tensor(int kind, int order, int ntl, int prec, const TensorArgs &a,
 // destination, whose two parts then go to memory separately (tile_shift's
 // figures).  Where rows keep their place in a line from row to row, a row is
 // therefore walked in whole lines of 16 slots from the line that holds its
-// first point, and the slots beside the row stay idle -- unless there would
-// be more of them than points: short rows share waves instead.  (Flat, and
-// with at most a quarter, a half, as many and twice as many idle slots: 2000
-// regions of 8-96 points per axis x 4 3.46, 3.33, 3.31, 3.30, 3.30 ms; step
-// of 432 boxes 1.320, 1.310, 1.303, 1.294, 1.298 ms.)
-void point_rows(PointArgs &a) {
+// first point, and the slots beside the row stay idle.  How many may is the
+// operator's: those that only move data take as many idle slots as points
+// (flat, and with at most a quarter, a half, as many and twice as many idle
+// slots: 2000 regions of 8-96 points per axis x 4 3.46, 3.33, 3.31, 3.30, 3.30
+// ms; step of 432 boxes 1.320, 1.310, 1.303, 1.294, 1.298 ms); the monotone
+// prolongation, up to 216 taps, a quarter (60 regions of 60x40x40 points, rows
+// 3 points into a line: 345 us against 426 flat; of 17x40x40, with 15 idle
+// slots a row: 328 against 186); the staggered operators and the higher-order
+// cell restrictions none, for each idle lane would have computed 27 to 216
+// terms (60 regions of 17x40x40 points: staggered prolongation 317 us in lines,
+// 178 flat, restriction 213 and 137; cell restriction of order 3 on 33x40x40
+// 89 and 75, of order 5 254 and 217; on 100x40x40 equal or slower in lines).
+static long long idle_slots(int op, long long points) {
+  switch (op) {
+  case PO_STAGGER:
+  case PO_RESTRICT_STAGGER:
+  case PO_RESTRICT_CC_O3:
+  case PO_RESTRICT_CC_O5: return -1;
+  case PO_MONO5: return points / 4;
+  }
+  return points;
+}
+
+void point_rows(int op, PointArgs &a) {
   const int s = (int)(reinterpret_cast<uintptr_t>(a.dst) / 8 % 16);
   const long long w = ((long long)s + a.n[0] + 15) / 16 * 16;
   // (regions of 2^30 slots and more stay flat: no fewer fit the 31-bit slot
   // numbers than points did)
-  const bool lines =
-      a.dj % 16 == 0 && a.dk % 16 == 0 && w <= 2LL * a.n[0] && w * a.n[1] < (1LL << 30) / std::max(1, a.n[2]);
+  const bool lines = a.dj % 16 == 0 && a.dk % 16 == 0 && w - a.n[0] <= idle_slots(op, a.n[0]) &&
+                     w * a.n[1] < (1LL << 30) / std::max(1, a.n[2]);
   a.sx = lines ? s : 0;
   a.nxp = lines ? (int)w : a.n[0];
 }
@@ -116,7 +134,7 @@ int launch_point(int op, const PointArgs &a0, hipStream_t s) {
     }
     return hipGetLastError() == hipSuccess ? 0 : -2;
   }
-  point_rows(a);
+  point_rows(op, a);
   const long long nxy = (long long)a.nxp * a.n[1];
   if (nxy <= 0 || a.n[2] <= 0 || nxy >= (1LL << 32) / 2)
     return -1;

@@ -124,9 +124,9 @@ inline int tiles_y(const TensorArgs &a, int cy) { return (a.n[1] + a.sy + 2 * cy
 // computes ntiles/zchunk (and sx, unless it is set) of a for a tile
 // configuration; returns block count
 long long tensor_tiles(TensorArgs &a, const TileCfg &cfg);
-// chooses the slots of a's rows (nxp, sx); the caller checks their number and
-// sets the divisors
-void point_rows(PointArgs &a);
+// chooses the slots of the rows of operator op on a (nxp, sx; not for TVD, which
+// counts coarse parents); the caller checks their number and sets the divisors
+void point_rows(int op, PointArgs &a);
 int launch_point(int op, const PointArgs &a, hipStream_t s);
 int launch_fill(double *dst, double v, size_t n, hipStream_t s);
 int launch_stream_copy(double *dst, const double *src, size_t n, hipStream_t s);

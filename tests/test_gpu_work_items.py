@@ -1,0 +1,83 @@
+"""How a batch cuts its transfers into work items: rows of operators that compute
+much per point have no idle slots, the segments of the eight XCDs hold equal
+numbers of items, classes that fit one round of workgroups take one each, and
+the tiles of a row are no more than they have to be."""
+import re
+
+import pytest
+
+cg = pytest.importorskip("carpet_amd")
+from carpet_amd.workloads import Box  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+V, C = cg.VERTEX_CENTERED, cg.CELL_CENTERED
+
+
+def _launches(b):
+    """items, grid, zchunk, points per item and mode of every launch"""
+    return [tuple(map(int, m)) for m in
+            re.findall(r"\] items (\d+) grid (\d+) zchunk (\d+) pt (\d+) wpc (-?\d+)", b.describe())]
+
+
+def _array(box, first=0, pad=16):
+    """A view whose element (0,0,0) lies `first` elements after a 128-byte line
+    and whose rows are padded to a multiple of `pad`.  Its storage is not large
+    enough: the batches here are built, not run."""
+    e = box.sizes()
+    return cg.DeviceArray.view(box, _base().ptr + 8 * first, ((e[0] + pad - 1) // pad * pad, e[1], e[2]))
+
+
+_own = []
+
+
+def _base():
+    if not _own:
+        _own.append(cg.DeviceArray(Box((0, 0, 0), (255, 0, 0), (1, 1, 1))))
+    return _own[0]
+
+
+def _prolong(b, n, cent, op, order, ntl=1, first=0, pad=16):
+    s, lo, h = (1, 2, 8) if cent == V else (2, 1, 8)
+    reg = Box((lo,) * 3, tuple(lo + (k - 1) * s for k in n), (s,) * 3)
+    up = tuple(u // (2 * s) for u in reg.upper)
+    src = Box((-2 * h,) * 3, tuple(2 * (u + h) for u in up), (2,) * 3) if cent == V else \
+        Box((2 - 4 * h,) * 3, tuple(2 + 4 * (u + h) for u in up), (4,) * 3)
+    d, a = _array(reg, first, pad), _array(src)
+    b.add(0, d, [a] * ntl, [0.0, -1.0, -2.0][:ntl], reg, reg, -0.5 if ntl > 1 else 0.0, op, cent, order, ntl - 1)
+
+
+def _restrict(b, n, first, op=cg.OP_LAGRANGE, cent=C):
+    if cent == C:
+        src = Box((1,) * 3, tuple(1 + 2 * (2 * k + 24) for k in n), (2,) * 3)
+        reg = Box((18,) * 3, tuple(18 + 4 * (k - 1) for k in n), (4,) * 3)
+    else:
+        src = Box((0,) * 3, tuple(2 * k + 24 for k in n), (1,) * 3)
+        reg = Box((8,) * 3, tuple(8 + 2 * (k - 1) for k in n), (2,) * 3)
+    b.add(0, _array(reg, first), [_array(src)], [0.0], reg, reg, 0.0, op, cent, 1, 0)
+
+
+@pytest.mark.parametrize("what,idle", [("stagger3", False), ("stagger2", False), ("restrict_stagger", False),
+                                       ("cc_o3", False), ("cc_o5", False), ("monotone", False), ("average", True)])
+def test_rows_of_costly_operators_have_no_idle_slots(what, idle):
+    """Rows of 17 points that begin 8 points into a line."""
+    n = (17, 40, 40)
+    cg.set_staggered_operators(True)
+    cg.set_restriction(what in ("cc_o3", "cc_o5"), 5 if what == "cc_o5" else 3)
+    try:
+        b = cg.Batch()
+        if what.startswith("stagger"):
+            _prolong(b, n, V, cg.OP_STAGGER111, int(what[-1]), first=8)
+        elif what == "monotone":
+            _prolong(b, n, V, cg.OP_LAGRANGE_MONOTONE, 5, first=8)
+        else:
+            st = what == "restrict_stagger"
+            _restrict(b, n, 8, cg.OP_STAGGER111 if st else cg.OP_LAGRANGE, V if st else C)
+        b.finalize()
+    finally:
+        cg.set_staggered_operators(False)
+        cg.set_restriction(False, 3)
+    items, _, _, pt, _ = _launches(b)[0]
+    slots = (32 if idle else 17) * 40 * 40
+    assert items == (slots + pt - 1) // pt, b.describe()
+    b.close()

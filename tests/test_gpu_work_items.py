@@ -81,3 +81,17 @@ def test_rows_of_costly_operators_have_no_idle_slots(what, idle):
     slots = (32 if idle else 17) * 40 * 40
     assert items == (slots + pt - 1) // pt, b.describe()
     b.close()
+
+
+def test_tvd_items_are_even_over_the_xcds():
+    """Regions of 172 items, which go to the XCDs in blocks of 16: the longest
+    of the eight segments, an eighth of the grid, holds at most 16 items more
+    than the mean."""
+    b = cg.Batch()
+    for _ in range(24):
+        _prolong(b, (112, 112, 112), C, cg.OP_TVD, 1)
+    b.finalize()
+    items, grid, _, _, wpc = _launches(b)[0]
+    assert items == 24 * 172 and wpc == -1
+    assert grid / 8 <= items / 8 + 16, b.describe()
+    b.close()

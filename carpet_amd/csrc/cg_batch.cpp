@@ -419,7 +419,8 @@ extern "C" int cg_batch_describe(const cg_batch *b, char *buf, size_t len) {
       const BatchLaunch &l = b->dev.launches[m];
       o << "phase " << l.phase << " [" << l.key << "] items " << l.nitems << " grid " << l.grid
         << " zchunk " << l.zchunk << " pt " << l.pt << " wpc " << l.wpc << " shape " << l.shape
-        << " ni " << l.ni;
+        << " ni " << l.ni
+        << (l.one_round ? " one round" : l.wpc == -1 ? " one per item" : l.wpc == -2 ? " fixed rounds" : " counters");
       if (j - i > 1)
         o << (b->dev.beside.size() != b->dev.launches.size() || b->dev.beside[i] ? " side by side"
                                                                                  : " in turn");

@@ -31,8 +31,9 @@ struct BatchLaunch {
                    // from counters (0 = resident capacity); -1 one
                    // workgroup per item; -2 resident capacity taking items
                    // in fixed rounds (tensor tiles)
-  bool one_round;  // tensor, wpc >= 0: the resident workgroups hold every item,
-                   // one each, and take it without counters
+  bool one_round;  // tensor, wpc 0 by default: the resident workgroups hold
+                   // every item, one workgroup each, and need no counters; in
+                   // turn with the phase's other launches
   int shape;       // tensor tile shape (0: 32 x 8 bases, 1: 16 x 16)
   int ni;          // grid mode, 256-point pointwise items: items per workgroup
   std::string key; // tuner cache key (class + box-size histogram bucket)

@@ -681,7 +681,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     // 642 us; 8 x 320^3 cell ENO<3> equal; 5 x 256^3 vertex ENO, 3 levels,
     // 378 against 323 us; 8 x 231x165x297 order 3, 2 levels, 240 against
     // 216 us.)  Regions of 2^20 points and up whose items fit one round of
-    // resident workgroups are persistent too, without counters (one_round).
+    // resident workgroups have a mode of their own (one_round, below).
     l.wpc = g.is_tensor && !g.small && median_pts >= (1LL << 25) ? 0 : -1;
     // tile shape: the class's (its regions were routed by shape)
     l.shape = !g.is_tensor ? 0 : g.small ? g.small : g.bigsh;
@@ -821,25 +821,24 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     // tiles share are fetched from HBM once, where striped over XCDs every
     // tile fetches them into its own L2.  A pointwise transfer with fewer
     // than 8 items gives each item to the least-loaded XCD.
-    int segb[9];
-    {
-      std::vector<Item> part[8];
+    const bool one = g.is_tensor && !g.small && median_pts >= (1LL << 20) && l.nitems <= full_grid;
+    auto split = [&](const std::vector<double> &w, std::vector<int> *part) {
       double load[8] = {0, 0, 0, 0, 0, 0, 0, 0};
       for (size_t m = 0; m + 1 < first.size(); ++m) {
         const int i0 = first[m], i1 = first[m + 1];
         if (g.is_tensor && i1 - i0 <= WHOLE_XCD_ITEMS) {
           const int x = (int)(std::min_element(load, load + 8) - load);
           for (int i = i0; i < i1; ++i) {
-            part[x].push_back(items[i]);
-            load[x] += cost[i];
+            part[x].push_back(i);
+            load[x] += w[i];
           }
           continue;
         }
         if (i1 - i0 < 8) {
           for (int i = i0; i < i1; ++i) {
             const int x = (int)(std::min_element(load, load + 8) - load);
-            part[x].push_back(items[i]);
-            load[x] += cost[i];
+            part[x].push_back(i);
+            load[x] += w[i];
           }
           continue;
         }
@@ -853,51 +852,87 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
           const int x0 = (int)(std::min_element(load, load + 8) - load);
           for (int i = i0; i < i1; ++i) {
             const int x = (x0 + (i - i0) / 16) % 8;
-            part[x].push_back(items[i]);
-            load[x] += cost[i];
+            part[x].push_back(i);
+            load[x] += w[i];
           }
           continue;
         }
         double total = 0;
         for (int i = i0; i < i1; ++i)
-          total += cost[i];
+          total += w[i];
         double acc = 0;
         int x = 0;
         for (int i = i0; i < i1; ++i) {
           // item i belongs to the part its cost midpoint falls in
-          const double mid = acc + 0.5 * cost[i];
+          const double mid = acc + 0.5 * w[i];
           while (x < 7 && mid >= total * (x + 1) / 8.0)
             ++x;
-          part[x].push_back(items[i]);
-          load[x] += cost[i];
-          acc += cost[i];
+          part[x].push_back(i);
+          load[x] += w[i];
+          acc += w[i];
         }
       }
-      items.clear();
+    };
+    std::vector<int> part[8];
+    split(cost, part);
+    // Classes of regions from 2^20 points whose items fit one round of resident
+    // workgroups: a segment longer than its XCD holds at once takes a second
+    // round, so the XCDs get equal numbers of items instead where that ends
+    // sooner (4 x 250x120x120 order 11, 3 levels, 256 items: 140 us with 36 on
+    // one XCD, 84 with 32 on each; 6 x 180^3 cell ENO<3>, 3 levels, whose second
+    // chunk is short: 562 us at equal cost, 600 at equal numbers).
+    if (one) {
+      auto end = [&](const std::vector<int> *pt) {
+        double e = 0;
+        for (int x = 0; x < 8; ++x) {
+          std::priority_queue<double, std::vector<double>, std::greater<double>> q;
+          for (int k = 0; k < full_grid / 8; ++k)
+            q.push(0.0);
+          for (int i : pt[x]) {
+            e = std::max(e, q.top() + cost[i]);
+            q.push(q.top() + cost[i]);
+            q.pop();
+          }
+        }
+        return e;
+      };
+      std::vector<int> even[8];
+      split(std::vector<double>(cost.size(), 1.0), even);
+      if (end(even) < 0.95 * end(part))
+        for (int x = 0; x < 8; ++x)
+          part[x].swap(even[x]);
+    }
+    int segb[9], longest = 1;
+    {
+      std::vector<Item> ordered;
+      ordered.reserve(items.size());
       segb[0] = 0;
       for (int x = 0; x < 8; ++x) {
-        items.insert(items.end(), part[x].begin(), part[x].end());
-        segb[x + 1] = (int)items.size();
+        for (int i : part[x])
+          ordered.push_back(items[i]);
+        segb[x + 1] = (int)ordered.size();
+        longest = std::max(longest, segb[x + 1] - segb[x]);
       }
+      items.swap(ordered);
       l.seg_off = append(segb, sizeof segb);
     }
     l.item_off = append(items.data(), items.size() * sizeof(Item));
     l.counter = (int)dev.launches.size();
-    if (l.wpc == -1 && !(tuned && tuned->count(l.key)) && g.is_tensor && !g.small &&
-        median_pts >= (1LL << 20) && l.nitems <= full_grid)
+    // one workgroup per item then, all of them resident, without counters (and
+    // the launch that clears them, 5-7 us); as it fills the GPU by itself it runs
+    // in turn with its phase's other classes (104x104x97 points and three thin
+    // faces, order 5, 3 levels: 19 us in turn, 34 side by side; 118x98x98 and 24
+    // of 20^3: 22 and 34).  A tuned class runs as its parameters say.
+    l.one_round = one && !(tuned && tuned->count(l.key));
+    if (l.one_round)
       l.wpc = 0;
-    // a persistent grid that holds every item at once needs no counters
-    l.one_round = l.wpc >= 0 && g.is_tensor && l.nitems <= full_grid;
     if (l.wpc == -1 || l.one_round) {
       // grid mode: 8 x the longest segment (in groups of ni items)
-      long long longest = 1;
-      for (int x = 0; x < 8; ++x)
-        longest = std::max<long long>(longest, segb[x + 1] - segb[x]);
       const int ni = (!g.is_tensor && l.pt == 256 && g.op != PO_TVD) ? l.ni : 1;
-      longest = (longest + ni - 1) / ni;
-      if (8 * longest > 0x7fffffffLL)
+      const long long groups = (longest + ni - 1) / ni;
+      if (8 * groups > 0x7fffffffLL)
         return set_error(CG_ERR_ARG, "too many work items for one launch");
-      l.grid = (int)(8 * longest);
+      l.grid = (int)(8 * groups);
     } else {
       const long long all = std::max(8, (l.nitems + 7) / 8 * 8);
       // persistent (counters or static rounds): a multiple of 8 workgroups

@@ -95,3 +95,18 @@ def test_tvd_items_are_even_over_the_xcds():
     assert items == 24 * 172 and wpc == -1
     assert grid / 8 <= items / 8 + 16, b.describe()
     b.close()
+
+
+@pytest.mark.parametrize("n,count,ntl,order", [((250, 120, 120), 4, 3, 11), ((250, 120, 120), 4, 3, 9)])
+def test_a_class_of_one_round_spreads_evenly(n, count, ntl, order):
+    """Items of about equal cost that just fit the resident workgroups: no XCD's
+    segment is longer than it holds at once."""
+    b = cg.Batch()
+    for _ in range(count):
+        _prolong(b, n, V, cg.OP_LAGRANGE, order, ntl, first=8)
+    b.finalize()
+    d = b.describe()
+    items, grid, _, _, wpc = _launches(b)[0]
+    assert wpc == 0 and "one round" in d, d
+    assert items <= grid < items + 8 * count, d
+    b.close()

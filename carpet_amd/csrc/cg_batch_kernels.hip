@@ -629,11 +629,13 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     l.prec = g.prec;
     // key of the tuner cache: kernel class + box-size histogram bucket
     // (log2 of the median destination points per transfer) + count bucket
-    long long median_pts = 0;
+    long long median_pts = 0, class_pts = 0;
     {
       std::vector<long long> pts;
       for (int m : g.members)
         pts.push_back(tr[m].dst_points());
+      for (long long n : pts)
+        class_pts += n;
       std::nth_element(pts.begin(), pts.begin() + pts.size() / 2, pts.end());
       median_pts = pts[pts.size() / 2];
       char key[128];
@@ -842,16 +844,21 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
           }
           continue;
         }
-        // TVD writes eight values per cell it reads, and writes best when the
-        // XCDs work close together: blocks of 16 items in turn (8 variables of
-        // 192^3 cells: slabs 987 us, single items 944, blocks of 16 919; the
-        // cell restriction back, which reads: 717, 750 and 757), from the
-        // XCD with the least work so far (24 regions of 56^3 cells, 172 items
-        // each: from XCD 0 every time 65.5 us, slabs 54.5)
-        if (g.op == PO_TVD && i1 - i0 >= 8 * 16) {
+        // TVD writes eight values per cell it reads, and writes to memory best
+        // when the XCDs work close together: blocks of 64 items in turn, from
+        // the XCD with the least work so far, where the class writes more than
+        // 1 GiB.  Below that much of it stays in the last-level cache, and slabs
+        // read each coarse plane on fewer XCDs.  (Slabs, and blocks of 16, 32
+        // and 64 items, us: 8 x 384^3 of 1 level 987, 890, 896, 894, of 3 levels
+        // 1403, 1380, 1381, 1353; 20 x 230^3, 1 level, 514, 476, 485, 487; 8 x
+        // 256^3, 1 level, 186, 219, 194, 189; 8 x 200^3, 2 levels, 101, 121, 101,
+        // 99.  The cell restriction back of 8 x 384^3, which reads: 717 in slabs,
+        // 757 in blocks of 16.)
+        constexpr int TVD_BLOCK = 64;
+        if (g.op == PO_TVD && class_pts > (1LL << 27) && i1 - i0 >= 8 * TVD_BLOCK) {
           const int x0 = (int)(std::min_element(load, load + 8) - load);
           for (int i = i0; i < i1; ++i) {
-            const int x = (x0 + (i - i0) / 16) % 8;
+            const int x = (x0 + (i - i0) / TVD_BLOCK) % 8;
             part[x].push_back(i);
             load[x] += w[i];
           }

@@ -83,17 +83,19 @@ def test_rows_of_costly_operators_have_no_idle_slots(what, idle):
     b.close()
 
 
-def test_tvd_items_are_even_over_the_xcds():
-    """Regions of 172 items, which go to the XCDs in blocks of 16: the longest
-    of the eight segments, an eighth of the grid, holds at most 16 items more
-    than the mean."""
+@pytest.mark.parametrize("n,count", [((112, 112, 112), 24), ((260, 256, 256), 8)])
+def test_tvd_items_are_even_over_the_xcds(n, count):
+    """Many medium regions, which are cut into slabs, and a gigabyte of large ones,
+    which go to the XCDs in blocks of 64 items: the longest of the eight
+    segments, an eighth of the grid, holds at most 64 items more than the mean."""
     b = cg.Batch()
-    for _ in range(24):
-        _prolong(b, (112, 112, 112), C, cg.OP_TVD, 1)
+    for _ in range(count):
+        _prolong(b, n, C, cg.OP_TVD, 1)
     b.finalize()
     items, grid, _, _, wpc = _launches(b)[0]
-    assert items == 24 * 172 and wpc == -1
-    assert grid / 8 <= items / 8 + 16, b.describe()
+    assert items == count * -(-n[0] * n[1] * n[2] // 8192)
+    assert wpc == -1
+    assert grid / 8 <= items / 8 + 64, b.describe()
     b.close()
 
 

@@ -252,16 +252,6 @@ struct Group {
   }
 };
 
-// Lanes a region keeps busy in tiles of shape sh: tiles x (planes + stencil
-// span) x (tile width) x (tile rows + span), the work of the window loads
-// and of the x- and y-passes.
-double tile_busy(const TensorArgs &a, int ntl, int prec, int span, int sh) {
-  int cx, cy, th;
-  tile_shape(ntl, prec, &cx, &cy, &th, sh);
-  return (double)tiles_x(a, cx, tile_shift(a, cx, prec ? 4 : 8)) * tiles_y(a, cy) * (a.nq[2] + span) * cx *
-         (cy + span);
-}
-
 int line_span(int kind, int order) {
   int span = 0;
   with_line(kind, order, [&](auto tag) -> int {
@@ -270,6 +260,17 @@ int line_span(int kind, int order) {
     return 0;
   });
   return span;
+}
+
+// Lanes a region keeps busy in tiles of shape sh: tiles x (planes + stencil
+// span) x (tile width) x (tile rows + span), the work of the window loads
+// and of the x- and y-passes.
+double tile_busy(const TensorArgs &a, int kind, int order, int ntl, int prec, int sh) {
+  const int span = line_span(kind, order);
+  int cx, cy, th;
+  tile_shape(ntl, prec, &cx, &cy, &th, sh);
+  return (double)tiles_x(a, cx, tile_shift(a, cx, prec ? 4 : 8, tile_cost(kind, order, ntl, prec))) * tiles_y(a, cy) *
+         (a.nq[2] + span) * cx * (cy + span);
 }
 
 // An FP64 region goes to the small tiles when they keep at most 1/1.3 of
@@ -288,9 +289,9 @@ int line_span(int kind, int order) {
 int small_tiles(const ProlongPlan &p, int ntl, int prec) {
   if (prec != CG_PREC_F64)
     return 0;
-  const int span = line_span(p.kind, p.order);
-  const double big = std::min(tile_busy(p.t, ntl, prec, span, 0), tile_busy(p.t, ntl, prec, span, 1));
-  const double b2 = tile_busy(p.t, ntl, prec, span, 2), b3 = tile_busy(p.t, ntl, prec, span, 3);
+  auto busy = [&](int sh) { return tile_busy(p.t, p.kind, p.order, ntl, prec, sh); };
+  const double big = std::min(busy(0), busy(1));
+  const double b2 = busy(2), b3 = busy(3);
   const int sh = CG_SLIM_TILES && p.t.nq[0] <= 4 && b3 < b2 ? 3 : 2;
   return (sh == 3 ? b3 : b2) * 1.3 <= big ? sh : 0;
 }
@@ -328,10 +329,10 @@ void merge_small_classes(const std::vector<Transfer> &tr, std::vector<Group> &pe
       seen |= 1 << (g.small ? g.small : g.bigsh);
       const TensorArgs &a = tr[j].pr.t;
       small = small && tr[j].dst_points() <= MERGE_POINTS;
-      const int span = line_span(g.kind, g.order);
-      busy += tile_busy(a, g.ntl, g.prec, span, g.small ? g.small : g.bigsh);
-      busy8 += tile_busy(a, g.ntl, g.prec, span, 2);
-      items += (long long)tiles_x(a, 8, tile_shift(a, 8, 8)) * tiles_y(a, 8) * ((a.nq[2] + 7) / 8);
+      busy += tile_busy(a, g.kind, g.order, g.ntl, g.prec, g.small ? g.small : g.bigsh);
+      busy8 += tile_busy(a, g.kind, g.order, g.ntl, g.prec, 2);
+      const int sx = tile_shift(a, 8, 8, tile_cost(g.kind, g.order, g.ntl, g.prec));
+      items += (long long)tiles_x(a, 8, sx) * tiles_y(a, 8) * ((a.nq[2] + 7) / 8);
     }
     if (small && __builtin_popcount((unsigned)seen) >= 3 && same.size() >= 128 &&
         items <= (busy8 <= 1.25 * busy ? 128LL : 32LL) * ncu)
@@ -357,6 +358,7 @@ TensorArgs tensor_desc(const BatchLaunch &l, const Transfer &t, int sx = -1) {
   tile_shape(l.ntl, l.prec, &cfg.cx, &cfg.cy, &th, l.shape);
   cfg.zchunk = l.zchunk;
   cfg.es = l.prec ? 4 : 8;
+  cfg.cost = tile_cost(l.kind, l.order, l.ntl, l.prec);
   (void)tensor_tiles(a, cfg);
   return a;
 }
@@ -555,9 +557,9 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
       // of the 3-level and the 2000-box hierarchies.
       g.bigsh = 0;
       if (!chosen && !g.small) {
-        const int span = line_span(tr[i].pr.kind, tr[i].pr.order);
-        const double b0 = tile_busy(tr[i].pr.t, cls_ntl[i], prec[i], span, 0);
-        const double b1 = tile_busy(tr[i].pr.t, cls_ntl[i], prec[i], span, 1);
+        const ProlongPlan &p = tr[i].pr;
+        const double b0 = tile_busy(p.t, p.kind, p.order, cls_ntl[i], prec[i], 0);
+        const double b1 = tile_busy(p.t, p.kind, p.order, cls_ntl[i], prec[i], 1);
         g.bigsh = b1 < 0.75 * b0 ? 1 : 0;
       }
       g.kind = tr[i].pr.kind;
@@ -733,7 +735,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
       // are few.  Near-ties go to the longer chunk (neighbouring tiles
       // then march through z together and share halo rows in L2).
       if (tile_cfg < 0 && !(tuned && tuned->count(l.key))) {
-        const int span = line_span(g.kind, g.order);
+        const int span = line_span(g.kind, g.order), tc = tile_cost(g.kind, g.order, g.ntl, g.prec);
         std::vector<double> mk;
         const int zcs[6] = {128, 64, 32, 16, 8, 4};
         for (int zc : zcs) {
@@ -743,7 +745,8 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
           for (int m : members) {
             const TensorArgs &a = tr[m].pr.t;
             const long long nxy =
-                (long long)tiles_x(a, cfg.cx, tile_shift(a, cfg.cx, g.prec ? 4 : 8)) * tiles_y(a, cfg.cy);
+                (long long)tiles_x(a, cfg.cx, tile_shift(a, cfg.cx, g.prec ? 4 : 8, tc)) *
+                tiles_y(a, cfg.cy);
             for (int z0 = 0; z0 < a.nq[2]; z0 += zc)
               for (long long t = 0; t < nxy; ++t) {
                 const double at = q.top();
@@ -885,7 +888,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     // Classes of regions from 2^20 points whose items fit one round of resident
     // workgroups: a segment longer than its XCD holds at once takes a second
     // round, so the XCDs get equal numbers of items instead where that ends
-    // sooner (4 x 250x120x120 order 11, 3 levels, 256 items: 140 us with 36 on
+    // sooner (4 x 250x120x120 order 11, 3 levels, 256 items: 147 us with 36 on
     // one XCD, 84 with 32 on each; 6 x 180^3 cell ENO<3>, 3 levels, whose second
     // chunk is short: 562 us at equal cost, 600 at equal numbers).
     if (one) {

@@ -16,17 +16,44 @@ namespace cg {
 // doubles from a line: 2.5-3.2 TB/s, against 5.5 TB/s aligned; 32 columns
 // 1.7-2.0 against 5.1, 16 columns 1.1-1.3 against 5.3.)  So the grid starts
 // at the line (or, for tiles of half a line, the half line) that holds the
-// region's first column, unless that takes noticeably more tiles.
-int tile_shift(const TensorArgs &a, int cx, int es) {
-  const int line = std::min(128 / es, 2 * cx);
-  const int s = (int)(reinterpret_cast<uintptr_t>(a.dst) / es % line);
+// region's first column -- where the rows keep their place in it from row to
+// row -- and where that takes more tiles of the same work, it depends on how
+// much a tile computes (tile_cost).  Batched, 12 regions of 250x200x200 points
+// 8 into a line, which are 4 tiles wide from the half line and 5 from the line,
+// and of 256x200x200 points 4 into a line, 4 tiles unaligned and 5 aligned:
+//   order 5, 1 level: line 244 us, half line 254; line 275, unaligned 362;
+//   order 5, 3 levels:     333,           290;         338,           365;
+//   cell ENO<3>, 3 levels: 1539,         1266;        1538,          1270;
+//   vertex ENO, 3 levels:   609,          499;         610,           505.
+// So cheap tiles take the line for up to a quarter more tiles, middling ones
+// the half line before that, and expensive ones never more tiles.
+int tile_cost(int kind, int order, int ntl, int prec) {
+  // multiplications per fine point and pass
+  const double taps = kind == LK_VLAG ? 0.5 * (order + 2) : kind == LK_CLAG ? order + 1
+                      : kind == LK_VENO ? 6 : order == 2 ? 8 : 16;
+  // FP32 storage passes the levels' combination, compensated sums take nine
+  // operations a tap
+  const double work = taps * (prec == 1 ? 1 : prec == 2 ? 9 * ntl : ntl);
+  return work <= 7 ? 0 : work <= 12 ? 1 : 2;
+}
+
+int tile_shift(const TensorArgs &a, int cx, int es, int cost) {
+  const int line = std::min(128 / es, 2 * cx), half = line / 2;
+  const int s = (int)(reinterpret_cast<uintptr_t>(a.dst) / es % line), h = s % half;
   const int n0 = tiles_x(a, cx, 0), n1 = tiles_x(a, cx, s);
-  return n1 <= n0 + n0 / 4 ? s : 0; // at most a quarter more (a half, an eighth: within 0.5% on the level steps)
+  const bool lines = a.dj % line == 0 && a.dk % line == 0;
+  const bool halves = half * es >= 64 && a.dj % half == 0 && a.dk % half == 0;
+  const bool more = lines && n1 <= n0 + n0 / 4;
+  if (lines && (n1 <= n0 || (cost == 0 && more)))
+    return s;
+  if (halves && tiles_x(a, cx, h) <= n0)
+    return h;
+  return cost <= 1 && more ? s : 0;
 }
 
 long long tensor_tiles(TensorArgs &a, const TileCfg &cfg) {
   if (a.sx < 0)
-    a.sx = tile_shift(a, cfg.cx, cfg.es);
+    a.sx = tile_shift(a, cfg.cx, cfg.es, cfg.cost);
   a.ntiles[0] = tiles_x(a, cfg.cx, a.sx);
   a.ntiles[1] = tiles_y(a, cfg.cy);
   a.zchunk = cfg.zchunk > 0 ? cfg.zchunk : a.nq[2];

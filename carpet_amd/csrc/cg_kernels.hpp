@@ -104,6 +104,7 @@ struct TileCfg {
   int cx, cy; // coarse bases per tile in x and y (fine tile 2cx x 2cy)
   int zchunk; // coarse bases per z chunk
   int es;     // bytes per element of the arrays
+  int cost;   // what a tile computes (tile_cost)
 };
 
 // ---- launchers (defined in cg_kernels.hip) --------------------------------
@@ -116,9 +117,11 @@ int launch_tensor_kind(int order, int ntl, int prec, const TensorArgs &a, const 
                        hipStream_t s);
 int launch_tensor(int kind, int order, int ntl, int prec, const TensorArgs &a,
                   const TileCfg &cfg, hipStream_t s);
+// how much the tiles of a line kind (LK_*) compute: 0 little, 1 middling, 2 much
+int tile_cost(int kind, int order, int ntl, int prec);
 // columns by which the tile grid of width 2 * cx starts before region r of a,
 // and the tiles along x that follow from it
-int tile_shift(const TensorArgs &a, int cx, int es);
+int tile_shift(const TensorArgs &a, int cx, int es, int cost);
 inline int tiles_x(const TensorArgs &a, int cx, int sx) { return (a.n[0] + sx + 2 * cx - 1) / (2 * cx); }
 inline int tiles_y(const TensorArgs &a, int cy) { return (a.n[1] + a.sy + 2 * cy - 1) / (2 * cy); }
 // computes ntiles/zchunk (and sx, unless it is set) of a for a tile

@@ -378,7 +378,7 @@ int launch_prolong(const ProlongPlan &pl, int prec, hipStream_t st) {
   } else if (pl.kind == PK_STAGGER) {
     r = launch_point(PO_STAGGER, pl.p, st);
   } else {
-    TileCfg cfg{0, 0, 0, pl.es};
+    TileCfg cfg{0, 0, 0, pl.es, tile_cost(pl.kind, pl.order, pl.ntl, prec)};
     // z chunks: at most 128 planes (tiles that march much further apart in
     // z stop sharing their halo rows through L2), halved down to 8 planes
     // while there are fewer than 2^18 threads (a full round of resident
@@ -391,7 +391,7 @@ int launch_prolong(const ProlongPlan &pl, int prec, hipStream_t st) {
     TensorArgs a = pl.t;
     int threads = 0;
     tile_shape(pl.ntl, prec, &cfg.cx, &cfg.cy, &threads);
-    const long long cols = (long long)tiles_x(a, cfg.cx, tile_shift(a, cfg.cx, cfg.es)) *
+    const long long cols = (long long)tiles_x(a, cfg.cx, tile_shift(a, cfg.cx, cfg.es, cfg.cost)) *
                            tiles_y(a, cfg.cy);
     int zc = std::min(a.nq[2], 128);
     while (zc > 4 && cols * ((a.nq[2] + zc - 1) / zc) * threads < (zc > 8 ? 1LL << 18 : 1LL << 16))

@@ -112,3 +112,24 @@ def test_a_class_of_one_round_spreads_evenly(n, count, ntl, order):
     assert wpc == 0 and "one round" in d, d
     assert items <= grid < items + 8 * count, d
     b.close()
+
+
+@pytest.mark.parametrize("cent,op,order,ntl,n,first,pad,tiles", [
+    (V, cg.OP_LAGRANGE, 5, 1, 250, 8, 16, 5),  # cheap: the line, for a quarter more tiles
+    (V, cg.OP_LAGRANGE, 5, 3, 250, 8, 16, 4),  # the half line
+    (V, cg.OP_LAGRANGE, 5, 3, 256, 4, 16, 5),  # unaligned but for one more tile
+    (C, cg.OP_ENO, 5, 3, 256, 4, 16, 4),  # expensive: no more tiles
+    (V, cg.OP_ENO, 3, 3, 256, 12, 16, 4),
+    (V, cg.OP_LAGRANGE, 5, 1, 250, 8, 1, 4),  # rows that lose their place in a line
+    (V, cg.OP_LAGRANGE, 3, 1, 250, 8, 2, 4),
+    (V, cg.OP_LAGRANGE, 5, 1, 248, 12, 8, 4),  # rows that keep their place in a half line
+])
+def test_tiles_along_x(cent, op, order, ntl, n, first, pad, tiles):
+    b = cg.Batch()
+    _prolong(b, (n, 112, 120), cent, op, order, ntl, first=first, pad=pad)
+    b.finalize(60)
+    d = b.describe()
+    assert "[tensor " in d, d
+    items = _launches(b)[0][0]
+    assert items in [tiles * rows * chunks for rows in (7, 8) for chunks in (1, 2)], d
+    b.close()

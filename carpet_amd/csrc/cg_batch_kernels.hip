@@ -484,31 +484,6 @@ void batch_device_free(BatchDevice &dev) {
   dev.ncounters = 0;
 }
 
-// Workgroups of fn that one CU holds at once, from the kernel's registers
-// and LDS and the device's per-CU LDS: each SIMD has 512 VGPRs per lane
-// (allocated in blocks of 8) and at most 8 waves; a workgroup's waves are
-// spread over the 4 SIMDs.  The runtime's occupancy query is the fallback
-// and the bound when it reports more.
-static int resident_per_cu(const void *fn, int threads, int dev) {
-  int api = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&api, fn, threads, 0) != hipSuccess)
-    api = 1;
-  hipFuncAttributes fa;
-  int lds_cu = 0;
-  if (hipFuncGetAttributes(&fa, fn) != hipSuccess ||
-      hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) !=
-          hipSuccess ||
-      fa.numRegs <= 0)
-    return std::max(1, api);
-  const int waves = (threads + 63) / 64;
-  const int per_simd = (waves + 3) / 4;
-  const int vgprs = (fa.numRegs + 7) / 8 * 8;
-  const int by_vgpr = std::min(8, 512 / vgprs) / per_simd;
-  const int by_lds = fa.sharedSizeBytes > 0 ? lds_cu / (int)fa.sharedSizeBytes : 32;
-  const int by_waves = 32 / waves;
-  return std::max({1, api, std::min({by_vgpr, by_lds, by_waves})});
-}
-
 static int ilog2(long long v) {
   int r = 0;
   while (v > 1) {

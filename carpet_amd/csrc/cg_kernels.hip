@@ -61,6 +61,80 @@ long long tensor_tiles(TensorArgs &a, const TileCfg &cfg) {
   return (long long)a.ntiles[0] * a.ntiles[1] * a.ntiles[2];
 }
 
+// Workgroups of fn that one CU holds at once, from the kernel's registers
+// and LDS and the device's per-CU LDS: each SIMD has 512 VGPRs per lane
+// (allocated in blocks of 8) and at most 8 waves; a workgroup's waves are
+// spread over the 4 SIMDs.  The runtime's occupancy query is the fallback
+// and the bound when it reports more.
+int resident_per_cu(const void *fn, int threads, int dev) {
+  int api = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&api, fn, threads, 0) != hipSuccess)
+    api = 1;
+  hipFuncAttributes fa;
+  int lds_cu = 0;
+  if (hipFuncGetAttributes(&fa, fn) != hipSuccess ||
+      hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) !=
+          hipSuccess ||
+      fa.numRegs <= 0)
+    return std::max(1, api);
+  const int waves = (threads + 63) / 64;
+  const int per_simd = (waves + 3) / 4;
+  const int vgprs = (fa.numRegs + 7) / 8 * 8;
+  const int by_vgpr = std::min(8, 512 / vgprs) / per_simd;
+  const int by_lds = fa.sharedSizeBytes > 0 ? lds_cu / (int)fa.sharedSizeBytes : 32;
+  const int by_waves = 32 / waves;
+  return std::max({1, api, std::min({by_vgpr, by_lds, by_waves})});
+}
+
+Resident resident_workgroups(const void *fn, int threads) {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    return {1, 256}; // no device: the launch that follows says so
+  return {resident_per_cu(fn, threads, dev), cus};
+}
+
+// z chunks of one call: at most 128 planes (tiles that march much further apart
+// in z stop sharing their halo rows through L2), halved while there are fewer
+// than 2^18 threads (a full round of resident workgroups), below 8 planes while
+// there are fewer than 2^16: a plane of a chunk takes 0.7 us on an idle GPU, so
+// chunks in parallel win although each reads the stencil's planes around it
+// again.  (Step of six calls, at least 16 against at least 8 and 4 planes: order
+// 5, 3 levels on 33^3 coarse points 60.6, 42.4 and 34.0 us; cell order 3, 2
+// levels on 75x61x90 93.0, 73.0 and 74.1 us, on 120^3 176.6, 163.2 and 170.6
+// us.)  Workgroups on one CU share its time, though, so below 16 planes a chunk
+// is halved only where that ends sooner: one call of 3 x 220^3 fine points takes
+// 78 us in chunks of 14 planes and 91 in chunks of 7 (order 7, 1 level; order 11,
+// 3 levels 290 and 390; cell order 5, 3 levels 149 and 180).  And chunks that
+// fill one round of resident workgroups are taken where they end sooner than
+// shorter ones that need a little more than a round, or longer ones that leave
+// CUs idle (order 7, 3 levels: 180^3 161 and 90 us; 256^3 199 and 174).
+int call_chunk(const TensorArgs &a, const TileCfg &cfg, int threads, int span, int per_cu, int cus) {
+  const long long cols =
+      (long long)tiles_x(a, cfg.cx, tile_shift(a, cfg.cx, cfg.es, cfg.cost)) * tiles_y(a, cfg.cy);
+  const long long round = (long long)per_cu * cus;
+  auto count = [&](int zc) { return cols * ((a.nq[2] + zc - 1) / zc); };
+  // planes in a row, a CU's time shared among its workgroups (fitted to orders
+  // 3 to 11 of all kinds, 66^3 to 300^3 fine points)
+  auto share = [&](long long n) { return n > 0 ? std::max(1.0, 0.25 + 0.6 * n / cus) : 0.0; };
+  auto time = [&](int zc) {
+    const long long n = count(zc);
+    return (n / round * share(round) + share(n % round)) * (zc + span);
+  };
+  auto half = [](int zc) { return (zc + 1) / 2; };
+  int zc = std::min(a.nq[2], 128);
+  while (zc > 16 && count(zc) * threads < (1LL << 18))
+    zc = half(zc);
+  while (zc > 4 && count(zc) * threads < (zc > 8 ? 1LL << 18 : 1LL << 16) && time(half(zc)) < time(zc))
+    zc = half(zc);
+  if (cols <= round && (count(zc) > round || count(zc) * threads < (1LL << 18))) {
+    const int fit = (int)((a.nq[2] + round / cols - 1) / (round / cols));
+    if (fit >= 4 && fit <= 128 && time(fit) < time(zc))
+      zc = fit;
+  }
+  return zc;
+}
+
 int launch_tensor(int kind, int order, int ntl, int prec, const TensorArgs &a,
                   const TileCfg &cfg, hipStream_t s) {
   if (prec < 0 || prec > 2 || (prec != 0 && fp64_only(kind)))

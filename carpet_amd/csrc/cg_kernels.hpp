@@ -127,6 +127,16 @@ inline int tiles_y(const TensorArgs &a, int cy) { return (a.n[1] + a.sy + 2 * cy
 // computes ntiles/zchunk (and sx, unless it is set) of a for a tile
 // configuration; returns block count
 long long tensor_tiles(TensorArgs &a, const TileCfg &cfg);
+// workgroups of kernel fn that one CU of device dev holds at once
+int resident_per_cu(const void *fn, int threads, int dev);
+// the same on the current device, and its CUs
+struct Resident {
+  int per_cu, cus;
+};
+Resident resident_workgroups(const void *fn, int threads);
+// planes per z chunk of one call's tiles (threads, stencil span and resident
+// workgroups of the kernel)
+int call_chunk(const TensorArgs &a, const TileCfg &cfg, int threads, int span, int per_cu, int cus);
 // chooses the slots of the rows of operator op on a (nxp, sx; not for TVD, which
 // counts coarse parents); the caller checks their number and sets the divisors
 void point_rows(int op, PointArgs &a);

@@ -379,25 +379,7 @@ int launch_prolong(const ProlongPlan &pl, int prec, hipStream_t st) {
     r = launch_point(PO_STAGGER, pl.p, st);
   } else {
     TileCfg cfg{0, 0, 0, pl.es, tile_cost(pl.kind, pl.order, pl.ntl, prec)};
-    // z chunks: at most 128 planes (tiles that march much further apart in
-    // z stop sharing their halo rows through L2), halved down to 8 planes
-    // while there are fewer than 2^18 threads (a full round of resident
-    // workgroups) and on to 4 below 2^16: a plane of a chunk takes 0.7 us
-    // on an idle GPU, so chunks in parallel win although each reads the
-    // stencil's planes around it again.  (Step of six calls, at least 16
-    // against at least 8 and 4 planes: order 5, 3 levels on 33^3 coarse
-    // points 60.6, 42.4 and 34.0 us; cell order 3, 2 levels on 75x61x90
-    // 93.0, 73.0 and 74.1 us, on 120^3 176.6, 163.2 and 170.6 us.)
-    TensorArgs a = pl.t;
-    int threads = 0;
-    tile_shape(pl.ntl, prec, &cfg.cx, &cfg.cy, &threads);
-    const long long cols = (long long)tiles_x(a, cfg.cx, tile_shift(a, cfg.cx, cfg.es, cfg.cost)) *
-                           tiles_y(a, cfg.cy);
-    int zc = std::min(a.nq[2], 128);
-    while (zc > 4 && cols * ((a.nq[2] + zc - 1) / zc) * threads < (zc > 8 ? 1LL << 18 : 1LL << 16))
-      zc = (zc + 1) / 2;
-    cfg.zchunk = zc;
-    r = launch_tensor(pl.kind, pl.order, pl.ntl, prec, a, cfg, st);
+    r = launch_tensor(pl.kind, pl.order, pl.ntl, prec, pl.t, cfg, st);
   }
   if (r == -1)
     return set_error(CG_ERR_ORDER, "no kernel for kind %d order %d ntl %d prec %d",

@@ -29,11 +29,15 @@ int launch_tensor_t(const TensorArgs &a0, const TileCfg &cfg0, hipStream_t s) {
   TileCfg cfg = cfg0;
   cfg.cx = T::CX;
   cfg.cy = T::CY;
+  constexpr int threads = tile_threads<NTL, 0, PR>();
+  const auto kernel = &k_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC>;
+  // of the kernel, the same on every gfx950
+  static const Resident res = resident_workgroups(reinterpret_cast<const void *>(kernel), threads);
+  cfg.zchunk = call_chunk(a, cfg, threads, L::TMAXALL - L::TMINALL, res.per_cu, res.cus);
   const long long nblk = tensor_tiles(a, cfg);
   if (nblk <= 0 || nblk > 0x7fffffffLL)
     return -1;
-  hipLaunchKernelGGL((k_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC>), dim3((unsigned)nblk),
-                     dim3(tile_threads<NTL, 0, PR>()), 0, s, a);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)nblk), dim3(threads), 0, s, a);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

@@ -607,12 +607,15 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     // key of the tuner cache: kernel class + box-size histogram bucket
     // (log2 of the median destination points per transfer) + count bucket
     long long median_pts = 0, class_pts = 0;
+    int levels = 1; // the most time levels that a member combines
     {
       std::vector<long long> pts;
       for (int m : g.members)
         pts.push_back(tr[m].dst_points());
       for (long long n : pts)
         class_pts += n;
+      for (int m : g.members)
+        levels = std::max(levels, !tr[m].is_prolong ? tr[m].pt.a.ntl : g.is_tensor ? tr[m].pr.ntl : tr[m].pr.p.ntl);
       std::nth_element(pts.begin(), pts.begin() + pts.size() / 2, pts.end());
       median_pts = pts[pts.size() / 2];
       char key[128];
@@ -831,12 +834,14 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
         // 1403, 1380, 1381, 1353; 20 x 230^3, 1 level, 514, 476, 485, 487; 8 x
         // 256^3, 1 level, 186, 219, 194, 189; 8 x 200^3, 2 levels, 101, 121, 101,
         // 99.  The cell restriction back of 8 x 384^3, which reads: 717 in slabs,
-        // 757 in blocks of 16.)
-        constexpr int TVD_BLOCK = 64;
-        if (g.op == PO_TVD && class_pts > (1LL << 27) && i1 - i0 >= 8 * TVD_BLOCK) {
+        // 757 in blocks of 16.)  One level above 2 GiB takes blocks of 16: 8 x
+        // 384^3 with that restriction after it 1649 us a step, 1679 in blocks of
+        // 64.
+        const int block = levels == 1 && class_pts > (1LL << 28) ? 16 : 64;
+        if (g.op == PO_TVD && class_pts > (1LL << 27) && i1 - i0 >= 8 * block) {
           const int x0 = (int)(std::min_element(load, load + 8) - load);
           for (int i = i0; i < i1; ++i) {
-            const int x = (x0 + (i - i0) / TVD_BLOCK) % 8;
+            const int x = (x0 + (i - i0) / block) % 8;
             part[x].push_back(i);
             load[x] += w[i];
           }

@@ -420,7 +420,8 @@ extern "C" int cg_batch_describe(const cg_batch *b, char *buf, size_t len) {
       o << "phase " << l.phase << " [" << l.key << "] items " << l.nitems << " grid " << l.grid
         << " zchunk " << l.zchunk << " pt " << l.pt << " wpc " << l.wpc << " shape " << l.shape
         << " ni " << l.ni
-        << (l.one_round ? " one round" : l.wpc == -1 ? " one per item" : l.wpc == -2 ? " fixed rounds" : " counters");
+        << (l.one_round ? " one round" : l.wpc == -1 ? " one per item" : l.wpc == -2 ? " fixed rounds" : " counters")
+        << (l.cols ? " columns" : "");
       if (j - i > 1)
         o << (b->dev.beside.size() != b->dev.launches.size() || b->dev.beside[i] ? " side by side"
                                                                                  : " in turn");

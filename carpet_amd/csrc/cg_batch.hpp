@@ -35,6 +35,8 @@ struct BatchLaunch {
                    // every item, one workgroup each, and need no counters; in
                    // turn with the phase's other launches
   int shape;       // tensor tile shape (0: 32 x 8 bases, 1: 16 x 16)
+  bool cols;       // tensor, FP32 storage: a thread owns two columns, not two
+                   // rows (every region's columns pair up)
   int ni;          // grid mode, 256-point pointwise items: items per workgroup
   std::string key; // tuner cache key (class + box-size histogram bucket)
   std::vector<int> members; // transfer indices in descriptor order

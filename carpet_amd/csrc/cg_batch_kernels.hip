@@ -684,6 +684,9 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
           l.shape = it->second.shape;
       }
     }
+    l.cols = g.is_tensor && g.prec == CG_PREC_MIXED && l.shape == 0 &&
+             std::all_of(g.members.begin(), g.members.end(),
+                         [&](int m) { return column_pairs(tensor_desc(l, tr[m])); });
     // persistent grid: resident workgroups per CU x CUs, a multiple of the
     // 8 XCDs
     int threads = 0;

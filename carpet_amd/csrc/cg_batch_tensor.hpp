@@ -26,7 +26,7 @@ constexpr int BATCH_PF = 1;
 
 // NTL: levels of the passes; NSRC: source levels (NSRC > NTL: combined at
 // the window store)
-template <class L, int NTL, int CX, int CY, int IPT, int PR, int NSRC>
+template <class L, int NTL, int CX, int CY, int IPT, int PR, int NSRC, bool COLS>
 __global__ __launch_bounds__(2 * CX * CY / IPT)
 __attribute__((amdgpu_waves_per_eu(persist_waves<L, NTL, CX, CY, IPT>()))) void k_persist_tensor(
     const TensorArgs *__restrict__ descs, const Item *__restrict__ items,
@@ -40,12 +40,12 @@ __attribute__((amdgpu_waves_per_eu(persist_waves<L, NTL, CX, CY, IPT>()))) void 
       return;
     const Item w = items[it];
     const TensorArgs a = descs[w.desc];
-    tensor_tile<L, NTL, CX, CY, IPT, PR, BATCH_PF, pipe_fits<L, NTL, CX, CY>(), NSRC>(a, (int)w.tile,
-                                                                                          smem);
+    tensor_tile<L, NTL, CX, CY, IPT, PR, BATCH_PF, pipe_fits<L, NTL, CX, CY>(), NSRC, COLS>(
+        a, (int)w.tile, smem);
   }
 }
 
-template <class L, int NTL, int CX, int CY, int IPT, int PR, int NSRC>
+template <class L, int NTL, int CX, int CY, int IPT, int PR, int NSRC, bool COLS>
 __global__ __launch_bounds__(2 * CX * CY / IPT)
 __attribute__((amdgpu_waves_per_eu(persist_waves<L, NTL, CX, CY, IPT>()))) void k_grid_tensor(
     const TensorArgs *__restrict__ descs, const Item *__restrict__ items,
@@ -56,22 +56,36 @@ __attribute__((amdgpu_waves_per_eu(persist_waves<L, NTL, CX, CY, IPT>()))) void 
     return;
   const Item w = items[it];
   const TensorArgs a = descs[w.desc];
-  tensor_tile<L, NTL, CX, CY, IPT, PR, BATCH_PF, pipe_fits<L, NTL, CX, CY>(), NSRC>(a, (int)w.tile, smem);
+  tensor_tile<L, NTL, CX, CY, IPT, PR, BATCH_PF, pipe_fits<L, NTL, CX, CY>(), NSRC, COLS>(a, (int)w.tile,
+                                                                                            smem);
+}
+
+// column pairs (tensor_tile's COLS) exist for the wide tiles of the FP32-storage,
+// FP64-arithmetic mode
+template <int PR, int SH> constexpr bool has_cols() { return PR == 1 && SH == 0; }
+
+template <class L, int NSRC, int PR, int SH, bool COLS>
+int batch_tensor_cols(const BatchLaunch &l, const TensorArgs *td, const Item *items,
+                      const int *seg, int *ctr, hipStream_t st) {
+  constexpr int NTL = pass_levels(NSRC, PR);
+  using T = TileShape<NTL, SH, PR>;
+  const dim3 block(tile_threads<NTL, SH, PR>());
+  if (l.wpc == -1 || l.one_round)
+    hipLaunchKernelGGL((k_grid_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC, COLS>), dim3(l.grid), block,
+                       0, st, td, items, seg);
+  else
+    hipLaunchKernelGGL((k_persist_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC, COLS>), dim3(l.grid),
+                       block, 0, st, td, items, seg, ctr, l.wpc == -2 ? 1 : 0);
+  return 0;
 }
 
 template <class L, int NSRC, int PR, int SH>
 int batch_tensor_go(const BatchLaunch &l, const TensorArgs *td, const Item *items,
                     const int *seg, int *ctr, hipStream_t st) {
-  constexpr int NTL = pass_levels(NSRC, PR);
-  using T = TileShape<NTL, SH, PR>;
-  const dim3 block(tile_threads<NTL, SH, PR>());
-  if (l.wpc == -1 || l.one_round)
-    hipLaunchKernelGGL((k_grid_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC>), dim3(l.grid), block,
-                       0, st, td, items, seg);
-  else
-    hipLaunchKernelGGL((k_persist_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC>), dim3(l.grid),
-                       block, 0, st, td, items, seg, ctr, l.wpc == -2 ? 1 : 0);
-  return 0;
+  if constexpr (has_cols<PR, SH>())
+    if (l.cols)
+      return batch_tensor_cols<L, NSRC, PR, SH, true>(l, td, items, seg, ctr, st);
+  return batch_tensor_cols<L, NSRC, PR, SH, false>(l, td, items, seg, ctr, st);
 }
 
 template <int KIND, int SH>
@@ -111,7 +125,10 @@ template <int KIND, int SH> const void *batch_tensor_fn_kind(const BatchLaunch &
       constexpr int NTL = pass_levels(NSRC, PR);
       using T = TileShape<NTL, SH, PR>;
       *threads = tile_threads<NTL, SH, PR>();
-      fn = reinterpret_cast<const void *>(&k_persist_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC>);
+      fn = reinterpret_cast<const void *>(&k_persist_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC, false>);
+      if constexpr (has_cols<PR, SH>())
+        if (l.cols)
+          fn = reinterpret_cast<const void *>(&k_persist_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC, true>);
     };
     auto by_prec = [&](auto ntlc) {
       if (l.prec == 0)

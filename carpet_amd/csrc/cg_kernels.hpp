@@ -124,6 +124,12 @@ int tile_cost(int kind, int order, int ntl, int prec);
 int tile_shift(const TensorArgs &a, int cx, int es, int cost);
 inline int tiles_x(const TensorArgs &a, int cx, int sx) { return (a.n[0] + sx + 2 * cx - 1) / (2 * cx); }
 inline int tiles_y(const TensorArgs &a, int cy) { return (a.n[1] + a.sy + 2 * cy - 1) / (2 * cy); }
+// the columns of FP32 region a (its sx chosen) pair up: it begins and ends at an
+// even column of its tiles, and the pairs are aligned in every row
+inline bool column_pairs(const TensorArgs &a) {
+  return a.sx % 2 == 0 && a.n[0] % 2 == 0 && a.dj % 2 == 0 && a.dk % 2 == 0 &&
+         (reinterpret_cast<uintptr_t>(a.dst) & 7) == 0;
+}
 // computes ntiles/zchunk (and sx, unless it is set) of a for a tile
 // configuration; returns block count
 long long tensor_tiles(TensorArgs &a, const TileCfg &cfg);

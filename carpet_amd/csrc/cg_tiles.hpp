@@ -142,9 +142,17 @@ template <int I, int N, class F> __device__ __forceinline__ bool unroll_while(F 
 // the window is stored (time interpolation before the spatial stencil, exact
 // by linearity up to rounding; the FP32-storage, FP64-arithmetic mode), so
 // the passes run once instead of once per level.
+// COLS: a thread with IPT = 2 owns two neighbouring fine columns of one base row
+// and not two base rows of one column, so that the y-pass reads LDS and the
+// emission writes memory in pairs; chosen where the regions' columns pair up
+// (column_pairs).  (FP32 storage, order 5, 3 levels, rows against columns: 8 x
+// 384^3 483 and 447 us, 12 x 128^3 32 and 30; where a region begins or ends
+// inside a pair, 8 x 384^3 753 and 963 us, 8 x 193^3 84 and 88.  In FP64 pairs
+// are 16-byte stores: 8 x 231x165x297 order 3, 179 us with rows, 195 with
+// columns.)
 // smem must be 16-byte aligned and hold TensorLds<..., PIPE ? 2 : 1>
 template <class L, int NTL, int CX, int CY, int IPT, int PR = 0, int PF = 1, int PIPE = 0,
-          int NSRC = NTL>
+          int NSRC = NTL, bool COLS = false>
 __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *smem) {
   using TS = typename Prec<PR>::S; // storage
   using CT = typename Prec<PR>::C; // arithmetic of the passes
@@ -153,14 +161,7 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
   using WT = std::conditional_t<TF, CT, TS>; // LDS window type
   constexpr int FX = 2 * CX;
   constexpr int NT = FX * CY / IPT;
-  // what a thread with IPT = 2 owns: two neighbouring fine columns of one base
-  // row where the arrays are FP32, so that the y-pass reads LDS and the
-  // emission writes memory in pairs (8 x 384^3, 3 levels: 633 against 595 us
-  // a pass; 8 x 198x178x158: 71.7 and 72.7; odd widths write a row's last
-  // line in two parts: 197 wide 72.5 and 77.7), else two base rows of one
-  // column (in FP64 pairs are 16-byte stores: 8 x 231x165x297 order 3, 179 us
-  // with rows, 195 with columns)
-  constexpr bool COLS = IPT == 2 && sizeof(TS) == 4;
+  static_assert(!COLS || (IPT == 2 && sizeof(TS) == 4), "column pairs: FP32 storage");
   constexpr int NC = COLS ? 2 : 1;     // columns of a thread
   constexpr int NQY = NT / (FX / NC);  // base rows of the threads' first items
   static_assert(IPT <= 2 && NQY * (IPT / NC) == CY, "tile rows must divide among threads");
@@ -217,7 +218,7 @@ __device__ __forceinline__ void tensor_tile(const TensorArgs &a, int b, double *
   const int gfx = tx * FX + fx - a.sx;
   const bool xin = gfx >= 0 && gfx < a.n[0];
   // COLS: pairs of columns are aligned in every row; the region begins or
-  // ends inside a pair
+  // ends inside a pair (new storage may have moved a region that paired up)
   const int px0 = tx * FX - a.sx; // the tile's first column
   const bool pairs = COLS && (((uintptr_t)a.dst + px0 * (long long)sizeof(TS)) & (2 * sizeof(TS) - 1)) == 0 &&
                      ((a.dj | a.dk) & 1) == 0;

@@ -592,8 +592,9 @@ int cg_batch_set_phase_mode(cg_batch *b, int phase, int mode);
    bytes of the device descriptor blob), then one line per launch (phase,
    class key, work items, grid, tile choice, grid mode, how its workgroups take
    items ("one per item", "one round": the same with every workgroup resident,
-   "fixed rounds" or "counters"); in phases of several launches "side by side"
-   or "in turn"); returns the full length */
+   "fixed rounds" or "counters"; "columns" where a thread owns two columns of
+   FP32 arrays); in phases of several launches "side by side" or "in turn");
+   returns the full length */
 int cg_batch_describe(const cg_batch *b, char *buf, size_t len);
 /* no reference counterpart: the launches of a finalized batch one at a
    time, for per-kernel timing -- their number, launch idx run on its own

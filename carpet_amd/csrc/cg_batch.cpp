@@ -192,7 +192,12 @@ int cg_batch_finalize(cg_batch *b, int tile_cfg) {
     return set_error(CG_ERR_STATE, "batch already finalized");
   b->tile_cfg = tile_cfg;
   b->shapes.clear();
-  int e = batch_device_build(b->dev, b->transfers, b->phase, b->prec, b->cls_ntl, b->shapes, tile_cfg, &b->tuned);
+  unsigned keep = 0;
+  for (const auto &m : b->phase_mode)
+    if (m.first >= 0 && m.first < 16)
+      keep |= 1u << m.first;
+  int e = batch_device_build(b->dev, b->transfers, b->phase, b->prec, b->cls_ntl, b->shapes, tile_cfg, &b->tuned,
+                             -1, keep);
   if (e)
     return e;
   index_launches(b);

@@ -92,11 +92,12 @@ struct BatchDevice {
 // shape of its launch class, chosen by the first build (an empty vector) and
 // kept by the later ones, so that the tuner's trials and rebuilds have the
 // same classes also after new storage has moved a region to another alignment;
-// only >= 0 builds launch `only` of the full build alone (the tuner's trials)
+// only >= 0 builds launch `only` of the full build alone (the tuner's trials);
+// keep_phases: bit mask of the phases whose small classes are not merged
 int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
                        const std::vector<int> &phase, const std::vector<int> &prec,
                        const std::vector<int> &cls_ntl, std::vector<char> &shapes, int tile_cfg,
-                       const TuneMap *tuned = nullptr, int only = -1);
+                       const TuneMap *tuned = nullptr, int only = -1, unsigned keep_phases = 0);
 // the descriptor array of launch l from the current transfers, in the
 // layout batch_device_build uploads (the per-step parameter path rewrites
 // it in place: same items, new time weights and array pointers)

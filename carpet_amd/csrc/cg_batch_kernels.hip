@@ -305,14 +305,15 @@ int small_tiles(const ProlongPlan &p, int ntl, int prec) {
 // 3, 2 levels 62 against 29 us, from a graph 45 against 33; a 3-level
 // hierarchy of 64^3 coarse points x 4 116 against 86 us, of 128^3 x 12, which
 // keeps its classes, 475 against 488 us; 432 boxes x 4 1.274 against 1.240
-// ms; 1000 regions of 8-60 points 626 against 598 us.)  Fewer than 128 regions
-// keep their classes, which a caller can run beside each other or in turn
+// ms; 1000 regions of 8-60 points 626 against 598 us.)  Fewer than 128 regions,
+// and the phases of the bit mask keep, which the caller has named a mode for,
+// keep their classes, so that they can run beside each other or in turn
 // (cg_batch_set_phase_mode).
 constexpr long long MERGE_POINTS = 1 << 18; // per region
-void merge_small_classes(const std::vector<Transfer> &tr, std::vector<Group> &per, int ncu) {
+void merge_small_classes(const std::vector<Transfer> &tr, std::vector<Group> &per, int ncu, unsigned keep) {
   std::vector<char> done(per.size(), 0);
   for (size_t i = 0; i < per.size(); ++i) {
-    if (done[i] || !per[i].is_tensor || per[i].prec != CG_PREC_F64)
+    if (done[i] || !per[i].is_tensor || per[i].prec != CG_PREC_F64 || (keep >> per[i].phase & 1))
       continue;
     std::vector<size_t> same;
     long long items = 0;
@@ -509,7 +510,7 @@ void batch_launch_descs(const BatchLaunch &l, const std::vector<Transfer> &tr, c
 int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
                        const std::vector<int> &phase, const std::vector<int> &prec,
                        const std::vector<int> &cls_ntl, std::vector<char> &shapes, int tile_cfg,
-                       const TuneMap *tuned, int only) {
+                       const TuneMap *tuned, int only, unsigned keep_phases) {
   batch_device_free(dev);
   // group transfers by (phase, kernel)
   const bool chosen = !shapes.empty();
@@ -560,7 +561,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
   if (he != hipSuccess)
     return hip_error(he, "hipDeviceGetAttribute");
   if (!chosen) {
-    merge_small_classes(tr, per, ncu);
+    merge_small_classes(tr, per, ncu, keep_phases);
     shapes.resize(tr.size());
   }
   for (size_t i = 0; i < tr.size(); ++i) {

@@ -586,7 +586,9 @@ int cg_batch_autotune(cg_batch *b, cg_stream_t stream, int reps,
    the other, -1 automatic: the tuner's choice, else side by side exactly
    when every launch of the phase runs one workgroup per item (a persistent
    launch fills the GPU by itself).  Any time; applies from the next
-   cg_batch_run or capture and drops a captured graph. */
+   cg_batch_run or capture and drops a captured graph.  From 128 regions on, a
+   phase's prolongations of small regions run as one launch, which has no mode
+   to choose, unless the phase's mode was set before cg_batch_finalize. */
 int cg_batch_set_phase_mode(cg_batch *b, int phase, int mode);
 /* human-readable summary: a totals line (transfers, launches, work items,
    bytes of the device descriptor blob), then one line per launch (phase,

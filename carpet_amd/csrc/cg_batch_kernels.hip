@@ -873,8 +873,9 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     // workgroups: a segment longer than its XCD holds at once takes a second
     // round, so the XCDs get equal numbers of items instead where that ends
     // sooner (4 x 250x120x120 order 11, 3 levels, 256 items: 147 us with 36 on
-    // one XCD, 84 with 32 on each; 6 x 180^3 cell ENO<3>, 3 levels, whose second
-    // chunk is short: 562 us at equal cost, 600 at equal numbers).
+    // one XCD, 84 with 32 on each; where the second round is of short chunks, equal
+    // cost is the better split: 6 x 180^3 cell ENO<3>, 3 levels, 562 us against
+    // 600; 12 x 160^3 FP32 storage, order 3, 50 against 54).
     if (one) {
       auto end = [&](const std::vector<int> *pt) {
         double e = 0;
@@ -892,7 +893,7 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
       };
       std::vector<int> even[8];
       split(std::vector<double>(cost.size(), 1.0), even);
-      if (end(even) < 0.95 * end(part))
+      if (end(even) < 0.8 * end(part))
         for (int x = 0; x < 8; ++x)
           part[x].swap(even[x]);
     }

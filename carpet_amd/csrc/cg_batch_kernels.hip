@@ -639,10 +639,13 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     }
     // TVD items count coarse parent cells (8 fine points each): 1024 cells
     // (8 variables of 192^3 -> 384^3: 0.98 ms against 1.00 ms with 512, 1.01
-    // with 2048 and 1.10 with 256); higher-order cell restrictions 1024
-    // points
-    else if (g.op == PO_TVD || g.op == PO_RESTRICT_CC_O3 || g.op == PO_RESTRICT_CC_O5)
+    // with 2048 and 1.10 with 256); cell restriction of order 3 1024 points, of
+    // order 5, 216 terms each, 512 (60 of 60x40x40 and of 100x40x40 points: 376
+    // and 605 us, against 408 and 653 with 1024)
+    else if (g.op == PO_TVD || g.op == PO_RESTRICT_CC_O3)
       l.pt = 1024;
+    else if (g.op == PO_RESTRICT_CC_O5)
+      l.pt = 512;
     // cell-centred restriction (8 children per point): 256 (the 384^3 ->
     // 192^3 restriction of the same set, at 256, 512, 1024 and 4096: 0.70,
     // 0.74, 0.76 and 0.79 ms)

@@ -531,12 +531,17 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
       // slower).  Per region rather than per class: 0.6% faster on 2000
       // regions of 8-96 points per axis, 1.8% and 1.2% on the level steps
       // of the 3-level and the 2000-box hierarchies.
+      // FP32 rows that lose their place in a 128-byte line from row to row take
+      // the wide tile from a smaller margin on: a narrow tile's row is one line
+      // long and goes out in two parts (6 x 256^3 in unpadded rows, order 9: 295
+      // us narrow, 156 wide, at 0.73 of the busy lanes).
       g.bigsh = 0;
       if (!chosen && !g.small) {
         const ProlongPlan &p = tr[i].pr;
+        const bool split = prec[i] == CG_PREC_MIXED && (p.t.dj % 32 || p.t.dk % 32);
         const double b0 = tile_busy(p.t, p.kind, p.order, cls_ntl[i], prec[i], 0);
         const double b1 = tile_busy(p.t, p.kind, p.order, cls_ntl[i], prec[i], 1);
-        g.bigsh = b1 < 0.75 * b0 ? 1 : 0;
+        g.bigsh = b1 < (split ? 0.6 : 0.75) * b0 ? 1 : 0;
       }
       g.kind = tr[i].pr.kind;
       g.order = tr[i].pr.order;

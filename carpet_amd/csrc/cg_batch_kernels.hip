@@ -667,12 +667,13 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     // persistent grid (its workgroups take the tiles in order, so
     // neighbouring tiles march through z together and share halo rows in
     // L2); other tensor classes and pointwise runs: one workgroup per item.
-    // (Measured, persistent against one per item: 4 x 512^3 order 5, 3
-    // levels 1.35 against 1.38 ms; 8 x 384^3 with FP32 storage 633 against
-    // 642 us; 8 x 320^3 cell ENO<3> equal; 5 x 256^3 vertex ENO, 3 levels,
-    // 378 against 323 us; 8 x 231x165x297 order 3, 2 levels, 240 against
-    // 216 us.)  Regions of 2^20 points and up whose items fit one round of
-    // resident workgroups have a mode of their own (one_round, below).
+    // (Persistent against one per item: 4 x 512^3 order 5, 3 levels, a pass
+    // among those of other arrays 1343 and 1377 us, alone 1381 and 1357; 8 x
+    // 384^3 with FP32 storage 597 and 602 us, alone 664 and 637; the same
+    // arrays again and again 1284 and 1243, 641 and 615; 4 x 384^3 cell
+    // ENO<3>, 3 levels, equal; below the line 5 x 256^3 vertex ENO, 3 levels,
+    // 378 and 323.)  Regions of 2^20 points and up whose items fit one round
+    // of resident workgroups have a mode of their own (one_round, below).
     l.wpc = g.is_tensor && !g.small && median_pts >= (1LL << 25) ? 0 : -1;
     // tile shape: the class's (its regions were routed by shape)
     l.shape = !g.is_tensor ? 0 : g.small ? g.small : g.bigsh;

@@ -879,13 +879,17 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
     std::vector<int> part[8];
     split(cost, part);
     // Classes of regions from 2^20 points whose items fit one round of resident
-    // workgroups: a segment longer than its XCD holds at once takes a second
-    // round, so the XCDs get equal numbers of items instead where that ends
-    // sooner (4 x 250x120x120 order 11, 3 levels, 256 items: 147 us with 36 on
-    // one XCD, 84 with 32 on each; where the second round is of short chunks, equal
-    // cost is the better split: 6 x 180^3 cell ENO<3>, 3 levels, 562 us against
-    // 600; 12 x 160^3 FP32 storage, order 3, 50 against 54).
-    if (one) {
+    // workgroups, one or two to a CU: a segment longer than its XCD holds at once
+    // takes a second round, so the XCDs get equal numbers of items instead where
+    // that ends sooner (4 x 250x120x120 order 11, 3 levels, 256 items: 147 us with
+    // 36 on one XCD, 84 with 32 on each; where the second round is of short chunks,
+    // equal cost is the better split: 6 x 180^3 cell ENO<3>, 3 levels, 562 us
+    // against 600).  Three and more workgroups to a CU share its rate, and the
+    // second round fills in as the first drains (equal cost and equal numbers, three
+    // to a CU, us: 6 x 67x145x161 vertex ENO<3>, 2 levels, 43 and 52; 9 x 139x66x209
+    // cell order 3, 2 levels, 54 and 59; 12 x 160^3 FP32 storage, order 3, 50 and 54.
+    // Of 34 such classes 5 were faster with equal numbers, by 9% at most.)
+    if (one && per_cu <= 2) {
       auto end = [&](const std::vector<int> *pt) {
         double e = 0;
         for (int x = 0; x < 8; ++x) {

@@ -114,6 +114,20 @@ def test_a_class_of_one_round_spreads_evenly(n, count, ntl, order):
     b.close()
 
 
+def test_a_class_of_one_round_with_three_workgroups_to_a_cu_keeps_equal_cost():
+    """Regions whose last z chunk is short: the segments of equal cost differ by
+    more items than there are regions."""
+    b = cg.Batch()
+    for _ in range(6):
+        _prolong(b, (67, 145, 161), V, cg.OP_ENO, 3, 2, first=8)
+    b.finalize()
+    d = b.describe()
+    items, grid, _, _, wpc = _launches(b)[0]
+    assert wpc == 0 and "one round" in d, d
+    assert grid >= items + 8 * 6, d
+    b.close()
+
+
 @pytest.mark.parametrize("cent,op,order,ntl,n,first,pad,tiles", [
     (V, cg.OP_LAGRANGE, 5, 1, 250, 8, 16, 5),  # cheap: the line, for a quarter more tiles
     (V, cg.OP_LAGRANGE, 5, 3, 250, 8, 16, 4),  # the half line

@@ -694,7 +694,13 @@ int batch_device_build(BatchDevice &dev, const std::vector<Transfer> &tr,
           l.shape = it->second.shape;
       }
     }
-    l.cols = g.is_tensor && g.prec == CG_PREC_MIXED && l.shape == 0 &&
+    // two columns a thread in narrow tiles from order 5 on and classes of 2^20
+    // points: 104 drawn classes of FP32 storage 2.5% faster, 70 of them by 1% or
+    // more, 2 slower (8 x 192x50x100 order 7 24.1 us with rows, 21.6 with columns;
+    // 10 x 68x34x205 order 9, 3 levels, 30.9 and 32.5); lower orders and smaller
+    // classes 0.3% slower (11 x 52x51x93 cell order 2, 2 levels, 8.8 and 9.3)
+    l.cols = g.is_tensor && g.prec == CG_PREC_MIXED &&
+             (l.shape == 0 || (l.shape == 1 && g.order >= 5 && class_pts >= (1LL << 20))) &&
              std::all_of(g.members.begin(), g.members.end(),
                          [&](int m) { return column_pairs(tensor_desc(l, tr[m])); });
     // persistent grid: resident workgroups per CU x CUs, a multiple of the

@@ -60,9 +60,11 @@ __attribute__((amdgpu_waves_per_eu(persist_waves<L, NTL, CX, CY, IPT>()))) void 
                                                                                             smem);
 }
 
-// column pairs (tensor_tile's COLS) exist for the wide tiles of the FP32-storage,
-// FP64-arithmetic mode
-template <int PR, int SH> constexpr bool has_cols() { return PR == 1 && SH == 0; }
+// column pairs (tensor_tile's COLS) exist for the FP32-storage, FP64-arithmetic
+// mode: wide tiles, and narrow ones of order 5 and more
+template <class L, int PR, int SH> constexpr bool has_cols() {
+  return PR == 1 && (SH == 0 || (SH == 1 && L::NTAP[1] >= 6));
+}
 
 template <class L, int NSRC, int PR, int SH, bool COLS>
 int batch_tensor_cols(const BatchLaunch &l, const TensorArgs *td, const Item *items,
@@ -82,7 +84,7 @@ int batch_tensor_cols(const BatchLaunch &l, const TensorArgs *td, const Item *it
 template <class L, int NSRC, int PR, int SH>
 int batch_tensor_go(const BatchLaunch &l, const TensorArgs *td, const Item *items,
                     const int *seg, int *ctr, hipStream_t st) {
-  if constexpr (has_cols<PR, SH>())
+  if constexpr (has_cols<L, PR, SH>())
     if (l.cols)
       return batch_tensor_cols<L, NSRC, PR, SH, true>(l, td, items, seg, ctr, st);
   return batch_tensor_cols<L, NSRC, PR, SH, false>(l, td, items, seg, ctr, st);
@@ -126,7 +128,7 @@ template <int KIND, int SH> const void *batch_tensor_fn_kind(const BatchLaunch &
       using T = TileShape<NTL, SH, PR>;
       *threads = tile_threads<NTL, SH, PR>();
       fn = reinterpret_cast<const void *>(&k_persist_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC, false>);
-      if constexpr (has_cols<PR, SH>())
+      if constexpr (has_cols<L, PR, SH>())
         if (l.cols)
           fn = reinterpret_cast<const void *>(&k_persist_tensor<L, NTL, T::CX, T::CY, T::IPT, PR, NSRC, true>);
     };

@@ -105,3 +105,28 @@ def test_call(n, k):
     cg.transfer_from_mixed(dd, ds, times, reg, reg, 1.0, cg.OP_LAGRANGE, V, 3, 0)
     cg.synchronize()
     _check(dd.download_padded(), exp, "call")
+
+
+@pytest.mark.parametrize("cent,order,ntl,n,k,columns", [(V, 7, 1, 66, 0, True), (C, 5, 2, 66, 2, True), (V, 5, 3, 66, 1, False),
+                                                        (V, 9, 1, 65, 0, False), (C, 4, 1, 66, 0, False)])
+def test_narrow_tiles_of_large_classes(cent, order, ntl, n, k, columns):
+    srcs, times, reg, box, exp = _case(cent, order, ntl, (n, 101, 161), k)
+    ds = [_dev(h) for h in srcs]
+    pad, count = _padded(box, 0)
+    own = cg.DeviceArray(cg.Box((0, 0, 0), (count + 31, 0, 0), (1, 1, 1)), dtype=np.float32, padext=(count + 32, 1, 1))
+    at = {s: cg.DeviceArray.view(box, own.ptr + 4 * s, pad, np.float32) for s in (0, 1)}
+    b = cg.Batch()
+    b.add(0, at[0], ds, times, reg, reg, 1 / 3 if ntl > 1 else 1.0, cg.OP_LAGRANGE, cent, order, ntl - 1, prec=cg.PREC_MIXED)
+    b.finalize()
+    d = b.describe()
+    assert "tensorN" in d and (" columns" in d) == columns, d
+    for s in (0, 1):
+        if s:
+            assert b.set_storage([(at[0], at[1])]) == 1
+        own.upload(np.full((1, 1, count + 32), np.nan, np.float32))
+        b.run()
+        cg.synchronize()
+        flat = own.download().ravel()
+        assert np.isnan(flat[:s]).all() and np.isnan(flat[s + count:]).all()
+        _check(flat[s:s + count].reshape(pad[::-1]), exp, f"at {s}")
+    b.close()
